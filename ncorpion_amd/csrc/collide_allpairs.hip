@@ -12,43 +12,21 @@
 #include <set>
 
 #include "ncg_internal.hpp"
+#include "collide_dev.hpp"
 
 #pragma clang fp contract(off)
 
 namespace {
 
-// Tile edge (bodies) of the upper-triangular tiling: 128, or 64 up to
-// CT_SMALL_N bodies, where 128-body tiles leave most SIMDs idle (n = 2000:
-// 136 workgroups of 128 lanes each walking 128 partners; with 64, 528
-// wavefronts walking 64).
-constexpr int CT_SMALL_N = 16384;
-__host__ __device__ constexpr int cand_tile(int n) { return n <= CT_SMALL_N ? 64 : 128; }
+// Tile edge (bodies) of the upper-triangular tiling of the all-pairs test,
+// used below NCG_CP_MIN bodies, where 128-body tiles leave most SIMDs idle
+// (n = 2000: 136 workgroups of 128 lanes each walking 128 partners; with 64,
+// 528 wavefronts walking 64).
+constexpr int CT = 64;
 
-// closest_approach's predicate (collision.c:112-137), same operations in the
-// same order.  The final time test keeps a relative slack of 2^-40 so the set
-// is a superset of the exact one whatever the last bit of sqrt/div; the host
-// re-evaluates every candidate exactly.
-__device__ inline bool approach_hit(double xa, double ya, double za, double vxa, double vya,
-                                    double vza, double ra, double xb, double yb, double zb,
-                                    double vxb, double vyb, double vzb, double rb, double dt)
-{
-    const double dx = xa - xb, dy = ya - yb, dz = za - zb;
-    const double dvx = vxa - vxb, dvy = vya - vyb, dvz = vza - vzb;
-    const double b = dx * dvx + dy * dvy + dz * dvz;
-    if (!(b < 0.0)) return false;
-    const double dr2 = dx * dx + dy * dy + dz * dz;
-    const double dv2 = dvx * dvx + dvy * dvy + dvz * dvz;
-    const double R = ra + rb;
-    const double disc = b * b + dv2 * (R * R - dr2);
-    if (!(disc > 0.0)) return false;
-    const double t = -(b + sqrt(disc)) / dv2;
-    return t <= dt + fabs(dt) * 9.094947017729282e-13;
-}
-
-template <int CT>
 __global__ __launch_bounds__(CT) void k_candidates(const DBody *__restrict__ b, int n,
                                                    const int32_t *__restrict__ ex, double dt,
-                                                   int ntiles, int2 *__restrict__ out,
+                                                   int2 *__restrict__ out,
                                                    unsigned long long cap,
                                                    unsigned long long *__restrict__ count)
 {
@@ -93,7 +71,6 @@ __global__ __launch_bounds__(CT) void k_candidates(const DBody *__restrict__ b, 
             if (slot < cap) out[slot] = make_int2(i, j);
         }
     }
-    (void)ntiles;
 }
 
 }  // namespace
@@ -102,17 +79,14 @@ ncg_status ncg_candidates_launch(ncg_ctx *ctx, const DBody *d_b, int32_t n, cons
                                  double dt, int2 *d_out, unsigned long long cap,
                                  unsigned long long *d_count, hipStream_t st)
 {
-    const int ct = cand_tile(n);
-    const int ntiles = (int)cdiv(n, ct);
+    if (n >= NCG_CP_MIN)
+        return ncg_cp_candidates_launch(ctx, d_b, n, d_ex, dt, d_out, cap, d_count, st);
+    const int ntiles = (int)cdiv(n, CT);
     const long nblk = (long)ntiles * (ntiles + 1) / 2;
     if (nblk == 0) return NCG_OK;
     ProfScope ps(ctx, st, "candidates");
-    if (ct == 64)
-        hipLaunchKernelGGL(k_candidates<64>, dim3((unsigned)nblk), dim3(64), 0, st, d_b, (int)n,
-                           d_ex, dt, ntiles, d_out, cap, d_count);
-    else
-        hipLaunchKernelGGL(k_candidates<128>, dim3((unsigned)nblk), dim3(128), 0, st, d_b, (int)n,
-                           d_ex, dt, ntiles, d_out, cap, d_count);
+    hipLaunchKernelGGL(k_candidates, dim3((unsigned)nblk), dim3(CT), 0, st, d_b, (int)n, d_ex, dt,
+                       d_out, cap, d_count);
     NCG_CHECK_LAUNCH();
     return NCG_OK;
 }
@@ -122,25 +96,14 @@ static ncg_status candidates_dev(ncg_ctx *ctx, const DBody *db, int32_t n, const
                                  double dt, std::vector<ncg_pair> &out)
 {
     hipStream_t st = ctx->stream;
-    const int ct = cand_tile(n);
-    const int ntiles = (int)cdiv(n, ct);
-    const long nblk = (long)ntiles * (ntiles + 1) / 2;
     unsigned long long cap = 1ull << 16;
     for (int attempt = 0; attempt < 2; ++attempt) {
         int2 *dout = dbuf<int2>(ctx, "cand", cap);
         unsigned long long *dcnt = dbuf<unsigned long long>(ctx, "cand_cnt", 1);
         if (!dout || !dcnt) return NCG_ERR_NOMEM;
         NCG_HIP(hipMemsetAsync(dcnt, 0, sizeof(unsigned long long), st));
-        {
-            ProfScope ps(ctx, st, "candidates");
-            if (ct == 64)
-                hipLaunchKernelGGL(k_candidates<64>, dim3((unsigned)nblk), dim3(64), 0, st, db,
-                                   (int)n, dex, dt, ntiles, dout, cap, dcnt);
-            else
-                hipLaunchKernelGGL(k_candidates<128>, dim3((unsigned)nblk), dim3(128), 0, st, db,
-                                   (int)n, dex, dt, ntiles, dout, cap, dcnt);
-            NCG_CHECK_LAUNCH();
-        }
+        const ncg_status r = ncg_candidates_launch(ctx, db, n, dex, dt, dout, cap, dcnt, st);
+        if (r != NCG_OK) return r;
         unsigned long long cnt = 0;
         NCG_HIP(hipMemcpyAsync(&cnt, dcnt, sizeof cnt, hipMemcpyDeviceToHost, st));
         NCG_HIP(hipStreamSynchronize(st));

@@ -9,6 +9,27 @@
 
 #pragma clang fp contract(off)
 
+// closest_approach's predicate (collision.c:112-137), same operations in the
+// same order.  The final time test keeps a relative slack of 2^-40 so the set
+// is a superset of the exact one whatever the last bit of sqrt/div; the host
+// re-evaluates every candidate exactly.
+__device__ inline bool approach_hit(double xa, double ya, double za, double vxa, double vya,
+                                    double vza, double ra, double xb, double yb, double zb,
+                                    double vxb, double vyb, double vzb, double rb, double dt)
+{
+    const double dx = xa - xb, dy = ya - yb, dz = za - zb;
+    const double dvx = vxa - vxb, dvy = vya - vyb, dvz = vza - vzb;
+    const double b = dx * dvx + dy * dvy + dz * dvz;
+    if (!(b < 0.0)) return false;
+    const double dr2 = dx * dx + dy * dy + dz * dz;
+    const double dv2 = dvx * dvx + dvy * dvy + dvz * dvz;
+    const double R = ra + rb;
+    const double disc = b * b + dv2 * (R * R - dr2);
+    if (!(disc > 0.0)) return false;
+    const double t = -(b + sqrt(disc)) / dv2;
+    return t <= dt + fabs(dt) * 9.094947017729282e-13;
+}
+
 // closest_approach on bodies a < c: hit when the pair approaches
 // (dr.dv < 0), meets (disc > 0) and meets within dt (t_c <= dt); ap receives
 // the positions at closest approach, heavier body first.

@@ -102,39 +102,6 @@ __device__ inline void box_axis(double lo, double hi, double &c, float &h)
 }
 
 // ---- order ------------------------------------------------------------------
-// Index along the Hilbert curve of a cell with 10-bit coordinates, after
-// J. Skilling, "Programming the Hilbert curve", AIP Conf. Proc. 707 (2004):
-// the coordinates are turned in place into the transposed index, whose bits
-// interleaved (x most significant) are the position along the curve.  Unlike
-// a Morton curve it has no jumps, so runs of keys are compact in space also
-// on a thin ring, where Morton runs straddle quadrant boundaries.
-__device__ inline unsigned hilbert10(unsigned x, unsigned y, unsigned z)
-{
-    unsigned X[3] = {x, y, z};
-    for (unsigned Q = 1u << 9; Q > 1; Q >>= 1) {
-        const unsigned P = Q - 1;
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            if (X[i] & Q) {
-                X[0] ^= P;  // invert
-            } else {        // exchange
-                const unsigned t = (X[0] ^ X[i]) & P;
-                X[0] ^= t;
-                X[i] ^= t;
-            }
-        }
-    }
-    X[1] ^= X[0];  // Gray encode
-    X[2] ^= X[1];
-    unsigned t = 0;
-    for (unsigned Q = 1u << 9; Q > 1; Q >>= 1)
-        if (X[2] & Q) t ^= Q - 1;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) X[i] ^= t;
-    return (expand10(X[0]) << 2) | (expand10(X[1]) << 1) | expand10(X[2]);
-}
-
-// One workgroup per system: bounding cube, largest radius, and the keys
 // (system << 30) | Hilbert index over the cube.
 __global__ __launch_bounds__(ENT) void k_ens_keys(const DBody *__restrict__ b,
                                                   const EnsSys *__restrict__ sys,
@@ -173,7 +140,7 @@ __global__ __launch_bounds__(ENT) void k_ens_keys(const DBody *__restrict__ b,
             v = v < 0 ? 0 : (v > 1023 ? 1023 : v);
             g[c] = (unsigned)v;
         }
-        key[S.off + k] = ((unsigned long long)blockIdx.x << 30) | hilbert10(g[0], g[1], g[2]);
+        key[S.off + k] = ((unsigned long long)blockIdx.x << 30) | hilbert<10>(g[0], g[1], g[2]);
         idx[S.off + k] = S.off + k;
     }
 }

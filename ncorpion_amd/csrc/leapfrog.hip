@@ -787,6 +787,9 @@ ncg_status leapfrog_run(ncg_ctx *ctx, ncg_body *d_bodies, int32_t n_in, int32_t 
         hipLaunchKernelGGL(k_lf_zero_u64, dim3(1), dim3(1), 0, st, cnt);
         ncg_status r = ncg_candidates_launch(ctx, b, n, ex, h, cand, cap, cnt, st);
         if (r != NCG_OK) return r;
+        if (n >= NCG_CP_MIN)
+            return ncg_cp_replay_launch(ctx, b, n, ex, d_did_collide, one_collision_only, cand, cnt,
+                                        cap, h, f, stat, st);
         return ncg_bf_replay_launch(ctx, b, ex, d_did_collide, one_collision_only, off, 1, cand,
                                     nullptr, cnt, cap, h, f, dirty, stat, st);
     };
@@ -1158,7 +1161,8 @@ ncg_status leapfrog_run(ncg_ctx *ctx, ncg_body *d_bodies, int32_t n_in, int32_t 
                         "collision replay capacity exceeded (flags %u: 1 = more than %u candidates, "
                         "2 = more than %d to decide, 4 = more than %d changed bodies in one pass); "
                         "results are not valid",
-                        hs[1], cap, NCG_REPLAY_RCAP, NCG_REPLAY_DCAP);
+                        hs[1], cap, n >= NCG_CP_MIN ? NCG_CP_EVENTS : NCG_REPLAY_RCAP,
+                        n >= NCG_CP_MIN ? NCG_CP_CHANGED : NCG_REPLAY_DCAP);
     return NCG_OK;
 }
 

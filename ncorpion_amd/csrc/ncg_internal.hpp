@@ -157,6 +157,24 @@ ncg_status ncg_candidates_launch(ncg_ctx *ctx, const DBody *d_b, int32_t n, cons
                                  double dt, int2 *d_out, unsigned long long cap,
                                  unsigned long long *d_count, hipStream_t st);
 
+// The same pass over spatial tiles for one system of NCG_CP_MIN bodies and more
+// (collide_tiled.hip): the candidates, and the replay over the tiles of the
+// last ncg_cp_candidates_launch with the same n on the same stream.  d_stat as
+// below.  From 8192 bodies: a 16-step run with collisions takes 210 us a step
+// there through the tiles against 220 with all pairs tested (387 against 789 at
+// 16,384; 192 against 168 at 6000, where the seven launches of the order cost
+// more than they save).
+constexpr int NCG_CP_MIN = 8192;
+constexpr int NCG_CP_EVENTS = 4096;   // candidates of a pass the tiled replay takes
+constexpr int NCG_CP_CHANGED = 1024;  // bodies changed in a pass it takes
+ncg_status ncg_cp_candidates_launch(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int32_t *d_ex,
+                                    double dt, int2 *d_out, unsigned long long cap,
+                                    unsigned long long *d_count, hipStream_t st);
+ncg_status ncg_cp_replay_launch(ncg_ctx *ctx, DBody *d_b, int32_t n, const int32_t *d_ex,
+                                int32_t *d_dc, int one_collision_only, const int2 *d_cand,
+                                const unsigned long long *d_count, unsigned cap, double dt,
+                                double f, unsigned *d_stat, hipStream_t st);
+
 // Device replay of a brute-force collision pass (replay.hip): one wavefront
 // per system (systems d_off[0..nsys]); candidates d_cand[0 .. *count) with
 // the count in d_count32 or d_count64; d_ex, d_dc may be null.  d_stat[0] +=

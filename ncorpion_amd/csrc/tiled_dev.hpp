@@ -32,6 +32,40 @@ __device__ inline unsigned expand10(unsigned v)
     return v;
 }
 
+// Index along the Hilbert curve of a cell with BITS-bit coordinates, after
+// J. Skilling, "Programming the Hilbert curve", AIP Conf. Proc. 707 (2004):
+// the coordinates are turned in place into the transposed index, whose bits
+// interleaved (x most significant) are the position along the curve.  Unlike
+// a Morton curve it has no jumps, so runs of keys are compact in space also
+// on a thin ring, where Morton runs straddle quadrant boundaries.
+template <int BITS>
+__device__ inline unsigned hilbert(unsigned x, unsigned y, unsigned z)
+{
+    unsigned X[3] = {x, y, z};
+    for (unsigned Q = 1u << (BITS - 1); Q > 1; Q >>= 1) {
+        const unsigned P = Q - 1;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            if (X[i] & Q) {
+                X[0] ^= P;  // invert
+            } else {        // exchange
+                const unsigned t = (X[0] ^ X[i]) & P;
+                X[0] ^= t;
+                X[i] ^= t;
+            }
+        }
+    }
+    X[1] ^= X[0];  // Gray encode
+    X[2] ^= X[1];
+    unsigned t = 0;
+    for (unsigned Q = 1u << (BITS - 1); Q > 1; Q >>= 1)
+        if (X[2] & Q) t ^= Q - 1;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) X[i] ^= t;
+    return (expand10(X[0]) << 2) | (expand10(X[1]) << 1) | expand10(X[2]);
+}
+
+// One workgroup per system: bounding cube, largest radius, and the keys
 template <class T>
 __device__ inline T block_reduce(T v, T *sh, int op /*0 min 1 max 2 sum*/)
 {

@@ -188,3 +188,50 @@ def test_replay_with_removed_and_created_bodies(ctx, seed):
     assert np.array_equal(bits(got.b[got.e != 0]), bits(ref.b[ref.e != 0]))
     kinds = {(7 * a + c) % 3 for a, c in ref.log}
     assert kinds == {0, 1, 2} and ref.largest >= n0  # removals, reuse and appends happened
+
+
+# The tiled pass takes 8192 bodies and more; one body in the last tile, the
+# finer cells above 16,384, holes, a body whose radius reaches every tile, and
+# a replay that runs out of room (replayed on the host).
+@pytest.mark.parametrize("n,radius,one,holes,cap", [
+    (8191, 1.5e-3, 0, False, None), (8192, 1.5e-3, 0, False, None), (8193, 1.5e-3, 1, True, None),
+    (16385, 5e-4, 0, True, None), (8200, 1.5e-3, 0, False, "8")])
+def test_tiled_pass_matches_oracle(monkeypatch, n, radius, one, holes, cap):
+    import torch
+    from ncorpion_amd import Context, ic
+    dt = 0.02
+    b = ic.disk(n, seed=n, mass=1e-8, radius=radius)
+    b[17, 7] = 0.03
+    b[5, 0:3] = 1e4  # one body far out
+    ex = None
+    if holes:
+        ex = (np.random.default_rng(n).uniform(size=n) > 0.1).astype(np.int32)
+    want, dc, pairs = orc.brute_force(b, dt, 1, 1.5, one, ex)
+    assert len(pairs) > 10
+    want[:, 0:3] += dt * want[:, 3:6]
+    on = slice(None) if ex is None else ex != 0
+    if cap is not None:
+        monkeypatch.setenv("NCG_REPLAY_CAP", cap)
+    ctx = Context(0)
+    try:
+        bt = torch.from_numpy(b).cuda()
+        ct = torch.zeros(8, dtype=torch.float64, device="cuda")
+        et = None if ex is None else torch.from_numpy(ex).cuda()
+        dct = torch.zeros(n, dtype=torch.int32, device="cuda")
+        # G = 0: the step is the collision pass and the drift.
+        got = ctx.leapfrog_dev(bt, ct, 1, dt, 0.0, 0.0, "fast64", 1.5, one, et, dct)
+        assert got == len(pairs)
+        assert np.array_equal(bits(bt.cpu().numpy()[on]), bits(want[on]))
+        # Candidates: those of the all-pairs predicate, a superset of the first
+        # hits of the reference's visits.
+        cand = ctx.collide_candidates(b, ex, dt)
+        first = [tuple(p) for p in pairs if orc.closest_approach(b, int(p[0]), int(p[1]), dt, ex)[0]]
+        assert set(first) <= {tuple(p) for p in cand}
+        bad = b.copy()
+        bad[3, 1], bad[9, 3], bad[11, 0] = np.nan, np.inf, -np.inf
+        clean = (np.ones(n, np.int32) if ex is None else ex.copy())
+        clean[[3, 9, 11]] = 0
+        assert np.array_equal(ctx.collide_candidates(bad, ex, dt),
+                              ctx.collide_candidates(b, clean, dt))
+    finally:
+        ctx.close()
