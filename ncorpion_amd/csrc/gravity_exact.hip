@@ -12,12 +12,11 @@
 // This translation unit is compiled with -ffp-contract=off: no FMA fusion.
 #include "ncg_internal.hpp"
 #include "exact_div.hpp"
+#include "exact_term.hpp"
 
 #pragma clang fp contract(off)
 
 namespace {
-
-constexpr int EX_T = 256;
 
 // physics.c:186-201 for body k at (X, Y, Z) and body j: D = sqrt(DX*DX +
 // DY*DY + DZ*DZ + soft*soft), D3 = D*D*D, term G m_j DX / D3, with DX formed
@@ -41,19 +40,97 @@ __device__ inline void exact_term(double X, double Y, double Z, double Rk, doubl
     }
 }
 
-// Central body from the host (cp, cx, cy, cz, mu) or, when dcen is given,
-// from a device record {x, y, z, vx, vy, vz, M, present}.
-__global__ __launch_bounds__(256) void k_grav_exact(const DBody *__restrict__ b, int n,
-                                                    const int32_t *__restrict__ ex, int cp,
-                                                    double cx, double cy, double cz, double mu,
-                                                    const double *__restrict__ dcen,
-                                                    double G, double s,
-                                                    const double *__restrict__ init,
-                                                    double *__restrict__ acc,
-                                                    double *__restrict__ cterm)
+// A workgroup takes EXP_B bodies k.  Waves 1..3 form the
+// terms of 192 bodies j at a time (one j per lane, EXP_B terms each) into LDS;
+// lanes 0 .. 3 EXP_B - 1 of wave 0 add the previous 192 terms, one component
+// of one body each, in j order.  A term to subtract is stored negated and a
+// skipped one as -0.0, so the sums are runs of additions: a - t and a + (-t)
+// are one operation, and a + (-0.0) is a for every a.  Block 0 forms CM_acc
+// the same way from the per-body reaction terms (physics.c:141-146 adds them
+// body by body), beside the other blocks.
+//
+// What bounds it: below ~5000 bodies the chain of dependent additions (5.7
+// clocks each), above it the FP64 issue of the terms (44 instructions when the
+// operands are in the window of exact_term.hpp).  EXP_B = 4 makes the two
+// halves of a chunk about equal (192 additions ~1100 clocks, 4 terms ~900).
+// One wavefront per body, its three summing lanes idle during the terms and
+// the other 61 during the sums, took 40 us at 2000 bodies and 2.27 ms at 20,011
+// (and CM_acc 13 and 101 us after it); this form takes 24 us and 1.16 ms with
+// CM_acc.  One body per lane, the form above 32,768 bodies before, took 25.7 ms
+// at 65,536 and 212 ms at 262,144, this one 10.9 and 171.  EXP_B = 2 takes 1.66 ms
+// at 20,011 (the summing wavefronts' share), 8 (two workgroups a CU by LDS) 1.17.
+constexpr int EXP_B = 4;
+constexpr int EXP_CH = 192;          // bodies j of a chunk
+constexpr int EXP_G = 8;             // pairs of terms the summing lanes read ahead
+constexpr int EXP_RS = EXP_CH + 2;   // row stride: the summing lanes read different banks
+
+// Body j of a term as read (skip: absent, or past n).
+struct ExpJ {
+    double x, y, z, m, R;
+    int skip;
+};
+
+__device__ inline ExpJ exp_load(const DBody *__restrict__ b, int n, const int32_t *__restrict__ ex,
+                                int j)
 {
-    __shared__ double tx[EX_T], ty[EX_T], tz[EX_T], tgm[EX_T], tr[EX_T];
-    __shared__ int te[EX_T];
+    ExpJ r;
+    const int jj = min(j, n - 1);
+    const DBody &q = b[jj];
+    r.x = q.x;
+    r.y = q.y;
+    r.z = q.z;
+    r.m = q.mass;
+    r.R = q.radius;
+    r.skip = j >= n;
+    if (ex) r.skip |= ex[jj] == 0;
+    return r;
+}
+
+// The window form for EXP_B bodies at once (their chains overlap): for j below
+// (LOWER, negated) or above all of them.  False, with nothing written, when an
+// operand is outside the window.  SOFT false: s is zero; with finite radii the
+// softening is then zero and adds nothing to r2.
+template <bool SOFT, bool LOWER>
+__device__ inline bool exp_window(const ExpJ &q, bool ok, double gm, const double *X,
+                                  const double *Y, const double *Z, const double *R, double s,
+                                  double (*row)[EXP_RS], int jl)
+{
+    double t[3][EXP_B], r2[EXP_B];
+#pragma unroll
+    for (int u = 0; u < EXP_B; ++u) {
+        t[0][u] = LOWER ? X[u] - q.x : q.x - X[u];
+        t[1][u] = LOWER ? Y[u] - q.y : q.y - Y[u];
+        t[2][u] = LOWER ? Z[u] - q.z : q.z - Z[u];
+        r2[u] = t[0][u] * t[0][u] + t[1][u] * t[1][u] + t[2][u] * t[2][u];
+        if (SOFT) {
+            const double soft = s * (R[u] + q.R);
+            r2[u] = r2[u] + soft * soft;
+        }
+        ok = ok && r2_ok(r2[u]);
+    }
+    if (!__all(ok || q.skip)) return false;
+    const bool holes = __any(q.skip);
+#pragma unroll
+    for (int u = 0; u < EXP_B; ++u) {
+        double v[3] = {gm * t[0][u], gm * t[1][u], gm * t[2][u]};
+        window_quotients<LOWER>(v, r2[u]);
+        if (holes && q.skip) v[0] = v[1] = v[2] = -0.0;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) row[3 * u + d][jl] = v[d];
+    }
+    return true;
+}
+
+template <bool SOFT>
+__global__ __launch_bounds__(256) void k_grav_exact_p(const DBody *__restrict__ b, int n,
+                                                      const int32_t *__restrict__ ex, int cp,
+                                                      double cx, double cy, double cz, double mu,
+                                                      const double *__restrict__ dcen, double G,
+                                                      double s, const double *__restrict__ init,
+                                                      double *__restrict__ acc, int cmblk,
+                                                      double *__restrict__ cm, NcgKickTail tail)
+{
+    __shared__ __align__(16) double st[2][3 * EXP_B][EXP_RS];
     if (dcen) {
         cp = dcen[7] != 0.0;
         cx = dcen[0];
@@ -61,303 +138,184 @@ __global__ __launch_bounds__(256) void k_grav_exact(const DBody *__restrict__ b,
         cz = dcen[2];
         mu = G * dcen[6];  // physics.c:131
     }
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool mine = k < n && (ex == nullptr || ex[k] != 0);
-    double X = 0., Y = 0., Z = 0., Rk = 0.;
-    double aX = 0., aY = 0., aZ = 0.;
-    if (mine) {
-        X = b[k].x;
-        Y = b[k].y;
-        Z = b[k].z;
-        Rk = b[k].radius;
-        const double mk = b[k].mass;
-        if (init) {  // the caller's start value (physics.c:121-172 beyond the point mass)
-            aX = init[3 * (size_t)k];
-            aY = init[3 * (size_t)k + 1];
-            aZ = init[3 * (size_t)k + 2];
-        } else if (cp) {
-            // physics.c:121-146
-            const double DX = X - cx, DY = Y - cy, DZ = Z - cz;
-            const double rk = sqrt(DX * DX + DY * DY + DZ * DZ);
-            const double r3 = rk * rk * rk;
-            aX = -mu * DX / r3;
-            aY = -mu * DY / r3;
-            aZ = -mu * DZ / r3;
-            cterm[3 * (size_t)k + 0] = G * mk * DX / r3;
-            cterm[3 * (size_t)k + 1] = G * mk * DY / r3;
-            cterm[3 * (size_t)k + 2] = G * mk * DZ / r3;
-        }
-    }
-    for (int base = 0; base < n; base += EX_T) {
-        const int jl = base + (int)threadIdx.x;
-        __syncthreads();
-        if (jl < n) {
-            const DBody q = b[jl];
-            tx[threadIdx.x] = q.x;
-            ty[threadIdx.x] = q.y;
-            tz[threadIdx.x] = q.z;
-            tgm[threadIdx.x] = G * q.mass;  // the reference's G*mp (physics.c:192)
-            tr[threadIdx.x] = q.radius;
-            te[threadIdx.x] = ex == nullptr ? 1 : (ex[jl] != 0);
-        } else {
-            te[threadIdx.x] = 0;
-        }
-        __syncthreads();
-        if (!mine) continue;
-        const int cnt = min(EX_T, n - base);
-        // Terms of four j at a time are formed independently (their square
-        // roots and divisions overlap), then added in j order: the sum is the
-        // reference's, skipped terms leave the accumulators untouched.
-        int jj = 0;
-        for (; jj + 4 <= cnt; jj += 4) {
-            double tX[4], tY[4], tZ[4];
-            bool use[4], low[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int j = base + jj + u;
-                use[u] = te[jj + u] && j != k;
-                low[u] = j < k;
-                exact_term(X, Y, Z, Rk, tx[jj + u], ty[jj + u], tz[jj + u], tr[jj + u],
-                           tgm[jj + u], s, low[u], tX[u], tY[u], tZ[u]);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if (!use[u]) continue;
-                if (low[u]) {
-                    aX -= tX[u];
-                    aY -= tY[u];
-                    aZ -= tZ[u];
-                } else {
-                    aX += tX[u];
-                    aY += tY[u];
-                    aZ += tZ[u];
-                }
-            }
-        }
-        for (; jj < cnt; ++jj) {
-            const int j = base + jj;
-            if (!te[jj] || j == k) continue;
-            const bool lower = j < k;
-            double tX, tY, tZ;
-            exact_term(X, Y, Z, Rk, tx[jj], ty[jj], tz[jj], tr[jj], tgm[jj], s, lower, tX, tY, tZ);
-            if (lower) {
-                aX -= tX;
-                aY -= tY;
-                aZ -= tZ;
-            } else {
-                aX += tX;
-                aY += tY;
-                aZ += tZ;
-            }
-        }
-    }
-    if (mine) {
-        acc[3 * (size_t)k + 0] = aX;
-        acc[3 * (size_t)k + 1] = aY;
-        acc[3 * (size_t)k + 2] = aZ;
-    }
-}
-
-// CM_acc as vector_field forms it: the per-body reaction terms added in body
-// order (physics.c:141-146 accumulates CM_acc body by body).  Waves 1..3
-// stage chunks of CMS_CH bodies' terms in LDS, a term of an absent body (or
-// past n) stored as -0.0, while lanes 0, 1, 2 of wave 0 add the x, y, z terms
-// of the previous chunk: a run of additions with no branch (a + (-0.0) is a
-// for every a, so a skipped body leaves the sum as it was).
-constexpr int CMS_CH = 1024;
-
-// The central body's presence comes from the device record dcen (its
-// present field) or, when dcen is null, from cp.
-__global__ __launch_bounds__(256) void k_cm_seq(const double *__restrict__ cterm, int n,
-                                                const int32_t *__restrict__ ex,
-                                                const double *__restrict__ dcen, int cp,
-                                                double *__restrict__ cm)
-{
-    // Rows padded by two doubles so that the three summing lanes read
-    // different banks.
-    __shared__ double st[2][3][CMS_CH + 2];
-    const int tid = threadIdx.x, w = tid >> 6;
-    if (dcen ? dcen[7] == 0.0 : cp == 0) {
+    // Role of the wavefront (0: the summing one).  It turns with the block, so
+    // that the summing wavefronts of a CU's blocks are not all on one SIMD.
+    const int turn = (int)((blockIdx.x >> 3) + (blockIdx.x >> 8));
+    const int w = __builtin_amdgcn_readfirstlane(((threadIdx.x >> 6) + turn) & 3);
+    const int lane = threadIdx.x & 63, tid = w * 64 + lane;
+    const bool sums = cmblk && blockIdx.x == 0;  // this block forms CM_acc
+    const int k0 = ((int)blockIdx.x - cmblk) * EXP_B;
+    const int nch = (n + EXP_CH - 1) / EXP_CH;
+    if (sums && tail.zero && tid == 0) *tail.zero = 0ull;
+    if (sums && !cp) {
         if (tid < 3) cm[tid] = 0.0;
         return;
     }
-    const int nch = (n + CMS_CH - 1) / CMS_CH;
-    auto stage = [&](int buf, int base) {
-        for (int q = tid - 64; q < CMS_CH; q += 192) {
-            const int k = base + q;
-            const bool on = k < n && (!ex || ex[k] != 0);
-            st[buf][0][q] = on ? cterm[3 * (size_t)k] : -0.0;
-            st[buf][1][q] = on ? cterm[3 * (size_t)k + 1] : -0.0;
-            st[buf][2][q] = on ? cterm[3 * (size_t)k + 2] : -0.0;
-        }
-    };
-    if (w > 0 && nch > 0) stage(0, 0);
-    __syncthreads();
-    double a = 0.0;
-    for (int c = 0; c < nch; ++c) {
-        if (w > 0) {
-            if (c + 1 < nch) stage((c + 1) & 1, (c + 1) * CMS_CH);
-        } else if (tid < 3) {
-            // Whole groups of 16 (the padding past n is -0.0).
-            const int len = (min(CMS_CH, n - c * CMS_CH) + 15) & ~15;
-            const double *row = st[c & 1][tid];
-            for (int q = 0; q < len; q += 16) {
+    if (w > 0) {
+        const int jl = tid - 64;
+        // The workgroup's bodies k (uniform).
+        double X[EXP_B], Y[EXP_B], Z[EXP_B], R[EXP_B];
+        bool kok = true;
+        if (!sums) {
 #pragma unroll
-                for (int u = 0; u < 16; ++u) a += row[q + u];
+            for (int u = 0; u < EXP_B; ++u) {
+                const DBody &q = b[min(k0 + u, n - 1)];
+                X[u] = q.x;
+                Y[u] = q.y;
+                Z[u] = q.z;
+                R[u] = q.radius;
+                kok = kok && coord_ok(X[u]) && coord_ok(Y[u]) && coord_ok(Z[u]) &&
+                      (SOFT || fabs(R[u]) < 1e100);
+            }
+        }
+        // The next chunk's records are in flight during the current terms.
+        ExpJ q = exp_load(b, n, ex, jl);
+        for (int c = 0; c < nch; ++c) {
+            const int j = c * EXP_CH + jl;
+            const ExpJ now = q;
+            if (c + 1 < nch) q = exp_load(b, n, ex, j + EXP_CH);
+            double(*row)[EXP_RS] = st[c & 1];
+            const double gm = G * now.m;  // the reference's G*mp (physics.c:192)
+            if (sums) {
+                double t[3] = {-0.0, -0.0, -0.0};
+                if (!now.skip) {
+                    // physics.c:121-146
+                    const double DX = now.x - cx, DY = now.y - cy, DZ = now.z - cz;
+                    const double rk = sqrt(DX * DX + DY * DY + DZ * DZ);
+                    const double r3 = rk * rk * rk;
+                    t[0] = gm * DX / r3;
+                    t[1] = gm * DY / r3;
+                    t[2] = gm * DZ / r3;
+                }
+                for (int d = 0; d < 3; ++d) row[d][jl] = t[d];
+            } else {
+                const int j0 = c * EXP_CH + (w - 1) * 64;
+                const bool ok = kok && coord_ok(now.x) && coord_ok(now.y) && coord_ok(now.z) &&
+                                gm_ok(gm) && (SOFT || fabs(now.R) < 1e100);
+                bool done = false;
+                if (j0 + 63 < k0) done = exp_window<SOFT, true>(now, ok, gm, X, Y, Z, R, s, row, jl);
+                else if (j0 >= k0 + EXP_B)
+                    done = exp_window<SOFT, false>(now, ok, gm, X, Y, Z, R, s, row, jl);
+                if (!done) {
+#pragma nounroll
+                    for (int u = 0; u < EXP_B; ++u) {
+                        const int k = k0 + u;
+                        const DBody &me = b[min(k, n - 1)];
+                        double t[3] = {-0.0, -0.0, -0.0};
+                        if (!now.skip && j != k) {
+                            exact_term(me.x, me.y, me.z, me.radius, now.x, now.y, now.z, now.R, gm,
+                                       s, j < k, t[0], t[1], t[2]);
+                            if (j < k)
+                                for (int d = 0; d < 3; ++d) t[d] = -t[d];
+                        }
+                        for (int d = 0; d < 3; ++d) row[3 * u + d][jl] = t[d];
+                    }
+                }
+            }
+            __syncthreads();
+        }
+        __syncthreads();
+        return;
+    }
+    const int u = lane / 3, d = lane - 3 * u;  // body and component of a summing lane
+    const int k = k0 + u;
+    const bool on = sums ? lane < 3 : u < EXP_B && k < n && (!ex || ex[k] != 0);
+    double a = 0.0;
+    if (!sums && on) {
+        if (init) {
+            a = init[3 * (size_t)k + d];
+        } else if (cp) {
+            // physics.c:121-146
+            const DBody me = b[k];
+            const double DX = me.x - cx, DY = me.y - cy, DZ = me.z - cz;
+            const double rk = sqrt(DX * DX + DY * DY + DZ * DZ);
+            const double r3 = rk * rk * rk;
+            const double D = d == 0 ? DX : d == 1 ? DY : DZ;
+            a = -mu * D / r3;
+        }
+    }
+    __syncthreads();
+    for (int c = 0; c < nch; ++c) {
+        if (on) {
+            const double2 *row = reinterpret_cast<const double2 *>(st[c & 1][sums ? lane : 3 * u + d]);
+            // 2 EXP_G terms are read while as many before them are added (all
+            // of a chunk: those past n are -0.0).
+            double2 x[EXP_G], y[EXP_G];
+#pragma unroll
+            for (int m = 0; m < EXP_G; ++m) x[m] = row[m];
+#pragma unroll
+            for (int i = EXP_G; i < EXP_CH / 2; i += 2 * EXP_G) {
+#pragma unroll
+                for (int m = 0; m < EXP_G; ++m) y[m] = row[i + m];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int m = 0; m < EXP_G; ++m) {
+                    a += x[m].x;
+                    a += x[m].y;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                if (i + EXP_G < EXP_CH / 2) {
+#pragma unroll
+                    for (int m = 0; m < EXP_G; ++m) x[m] = row[i + EXP_G + m];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int m = 0; m < EXP_G; ++m) {
+                    a += y[m].x;
+                    a += y[m].y;
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
         __syncthreads();
     }
-    if (tid < 3) cm[tid] = a;
-}
-
-// Small n: one wavefront per body k.  The lanes form the terms of 64 bodies j
-// at a time (exact_term, as k_grav_exact does), and lanes 0, 1, 2 add the x,
-// y, z terms in j order: the same sums, with 64 lanes forming the terms of one
-// body instead of one lane forming them all.  A term to subtract is stored
-// negated and a skipped one as -0.0, so the sum is a run of additions:
-// a - t and a + (-t) are one operation, and a + (-0.0) is a for every a.
-constexpr int EXW_MAX = 32768;  // bodies up to which the wavefront-per-body form is used
-
-__global__ __launch_bounds__(256) void k_grav_exact_w(const DBody *__restrict__ b, int n,
-                                                      const int32_t *__restrict__ ex, int cp,
-                                                      double cx, double cy, double cz, double mu,
-                                                      const double *__restrict__ dcen,
-                                                      double G, double s,
-                                                      const double *__restrict__ init,
-                                                      double *__restrict__ acc,
-                                                      double *__restrict__ cterm)
-{
-    __shared__ double st[4][3][64];
-    if (dcen) {
-        cp = dcen[7] != 0.0;
-        cx = dcen[0];
-        cy = dcen[1];
-        cz = dcen[2];
-        mu = G * dcen[6];  // physics.c:131
+    if (!on) return;
+    if (sums) {
+        cm[lane] = a;
+        if (tail.kcen) tail.kcen[3 + lane] += tail.h * a;
+    } else {
+        acc[3 * (size_t)k + d] = a;
+        if (tail.kb) (&tail.kb[k].vx)[d] += tail.h * a;
     }
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int k = blockIdx.x * 4 + w;
-    if (k >= n || (ex != nullptr && ex[k] == 0)) return;  // the whole wavefront
-    const DBody me = b[k];
-    const double X = me.x, Y = me.y, Z = me.z, Rk = me.radius;
-    double a = 0.;  // component `lane` (lanes 0..2)
-    if (init) {
-        if (lane < 3) a = init[3 * (size_t)k + lane];
-    } else if (cp) {
-        // physics.c:121-146
-        const double DX = X - cx, DY = Y - cy, DZ = Z - cz;
-        const double rk = sqrt(DX * DX + DY * DY + DZ * DZ);
-        const double r3 = rk * rk * rk;
-        const double aX = -mu * DX / r3, aY = -mu * DY / r3, aZ = -mu * DZ / r3;
-        a = lane == 0 ? aX : lane == 1 ? aY : aZ;
-        if (lane == 0) {
-            cterm[3 * (size_t)k + 0] = G * me.mass * DX / r3;
-            cterm[3 * (size_t)k + 1] = G * me.mass * DY / r3;
-            cterm[3 * (size_t)k + 2] = G * me.mass * DZ / r3;
-        }
-    }
-    // The next group's records are loaded before the current group is
-    // summed, so their latency overlaps the ordered additions.
-    DBody q = {};
-    int e = 0;
-    if (lane < n) {
-        q = b[lane];
-        e = ex == nullptr ? 1 : ex[lane];
-    }
-    for (int base = 0; base < n; base += 64) {
-        const int j = base + lane;
-        double tX = -0.0, tY = -0.0, tZ = -0.0;
-        if (j < n && j != k && e != 0) {
-            const bool lower = j < k;
-            exact_term(X, Y, Z, Rk, q.x, q.y, q.z, q.radius, G * q.mass, s, lower, tX, tY, tZ);
-            if (lower) {
-                tX = -tX;
-                tY = -tY;
-                tZ = -tZ;
-            }
-        }
-        const int jn = j + 64;
-        if (jn < n) {
-            q = b[jn];
-            e = ex == nullptr ? 1 : ex[jn];
-        }
-        st[w][0][lane] = tX;
-        st[w][1][lane] = tY;
-        st[w][2][lane] = tZ;
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        if (lane < 3) {
-            const double *row = st[w][lane];
-            for (int g = 0; g < 64; g += 16) {
-                double v[16];
-#pragma unroll
-                for (int i = 0; i < 16; ++i) v[i] = row[g + i];
-#pragma unroll
-                for (int i = 0; i < 16; ++i) a += v[i];
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    }
-    if (lane < 3) acc[3 * (size_t)k + lane] = a;
 }
 
 }  // namespace
 
-// Launches the exact kernel; cterm (3n) receives the per-body central
-// reaction terms when central->present.
-ncg_status ncg_grav_exact_launch(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int32_t *d_ex,
-                                 const ncg_central *c, double G, double soft, double *d_acc,
-                                 double *d_cterm, hipStream_t st, const double *d_init)
+// The field, and with cm (null: not wanted) CM_acc summed in body order.
+static ncg_status exact_launch(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int32_t *d_ex,
+                               const ncg_central *c, const double *d_cen, double G, double soft,
+                               const double *d_init, double *d_acc, double *d_cm_acc,
+                               const NcgKickTail &tail, hipStream_t st)
 {
     const int cp = (c && c->present) ? 1 : 0;
+    const double cx = cp ? c->x : 0.0, cy = cp ? c->y : 0.0, cz = cp ? c->z : 0.0;
     const double mu = cp ? G * c->mass : 0.0;  // physics.c:131
-    if (n <= EXW_MAX)
-        hipLaunchKernelGGL(k_grav_exact_w, dim3(cdiv(n, 4)), dim3(256), 0, st, d_b, (int)n, d_ex, cp,
-                           cp ? c->x : 0.0, cp ? c->y : 0.0, cp ? c->z : 0.0, mu,
-                           (const double *)nullptr, G, soft, d_init, d_acc, d_cterm);
+    const int cmblk = d_cm_acc ? 1 : 0;
+    const dim3 grid(cmblk + cdiv(n, EXP_B));
+    if (soft != 0.0)
+        hipLaunchKernelGGL(k_grav_exact_p<true>, grid, dim3(256), 0, st, d_b, (int)n, d_ex, cp, cx,
+                           cy, cz, mu, d_cen, G, soft, d_init, d_acc, cmblk, d_cm_acc, tail);
     else
-        hipLaunchKernelGGL(k_grav_exact, dim3(cdiv(n, 256)), dim3(256), 0, st, d_b, (int)n, d_ex, cp,
-                           cp ? c->x : 0.0, cp ? c->y : 0.0, cp ? c->z : 0.0, mu,
-                           (const double *)nullptr, G, soft, d_init, d_acc, d_cterm);
+        hipLaunchKernelGGL(k_grav_exact_p<false>, grid, dim3(256), 0, st, d_b, (int)n, d_ex, cp, cx,
+                           cy, cz, mu, d_cen, G, soft, d_init, d_acc, cmblk, d_cm_acc, tail);
     NCG_CHECK_LAUNCH();
     return NCG_OK;
 }
 
-// The same with the central body in a device record (8 doubles), and
-// CM_acc summed on the device in the reference's order.
+ncg_status ncg_grav_exact_launch(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int32_t *d_ex,
+                                 const ncg_central *c, double G, double soft, double *d_acc,
+                                 double *d_cm_acc, hipStream_t st, const double *d_init)
+{
+    return exact_launch(ctx, d_b, n, d_ex, c, nullptr, G, soft, d_init, d_acc, d_cm_acc,
+                        NcgKickTail{}, st);
+}
+
+// The same with the central body in a device record (8 doubles).
 ncg_status ncg_grav_exact_dev(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int32_t *d_ex,
                               const double *d_cen, double G, double soft, double *d_acc,
-                              double *d_cterm, double *d_cm_acc, hipStream_t st)
+                              double *d_cm_acc, const NcgKickTail &tail, hipStream_t st)
 {
-    {
-        ProfScope ps(ctx, st, "exact");
-        if (n <= EXW_MAX)
-            hipLaunchKernelGGL(k_grav_exact_w, dim3(cdiv(n, 4)), dim3(256), 0, st, d_b, (int)n, d_ex,
-                               0, 0.0, 0.0, 0.0, 0.0, d_cen, G, soft, (const double *)nullptr, d_acc,
-                               d_cterm);
-        else
-            hipLaunchKernelGGL(k_grav_exact, dim3(cdiv(n, 256)), dim3(256), 0, st, d_b, (int)n, d_ex,
-                               0, 0.0, 0.0, 0.0, 0.0, d_cen, G, soft, (const double *)nullptr, d_acc,
-                               d_cterm);
-        NCG_CHECK_LAUNCH();
-    }
-    if (d_cm_acc) {
-        hipLaunchKernelGGL(k_cm_seq, dim3(1), dim3(256), 0, st, d_cterm, (int)n, d_ex, d_cen, 0,
-                           d_cm_acc);
-        NCG_CHECK_LAUNCH();
-    }
-    return NCG_OK;
-}
-
-// CM_acc from the per-body terms d_cterm of an exact evaluation with the
-// central body given on the host (cp: present), summed in body order.
-ncg_status ncg_cm_seq_launch(ncg_ctx *ctx, const double *d_cterm, int32_t n, const int32_t *d_ex,
-                             int cp, double *d_cm_acc, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_cm_seq, dim3(1), dim3(256), 0, st, d_cterm, (int)n, d_ex,
-                       (const double *)nullptr, cp, d_cm_acc);
-    NCG_CHECK_LAUNCH();
-    return NCG_OK;
+    ProfScope ps(ctx, st, "exact");
+    return exact_launch(ctx, d_b, n, d_ex, nullptr, d_cen, G, soft, nullptr, d_acc, d_cm_acc, tail,
+                        st);
 }

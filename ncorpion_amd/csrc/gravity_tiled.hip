@@ -873,20 +873,13 @@ ncg_status ncg_gravity_dev_impl(ncg_ctx *ctx, const DBody *d_b, int32_t n, const
     if (n == 0) return NCG_OK;
     const int cp = (c && c->present) ? 1 : 0;
     if (prec == NCG_F64_EXACT) {
-        double *cterm = d_cterm;
-        if (cp && !cterm) {
-            cterm = dbuf<double>(ctx, "cterm", 3 * (size_t)n);
-            if (!cterm) return NCG_ERR_NOMEM;
-        }
         ncg_status r;
         {
             ProfScope ps(ctx, st, "exact");
-            r = ncg_grav_exact_launch(ctx, d_b, n, d_ex, c, G, soft, d_acc, cterm, st, d_init);
+            r = ncg_grav_exact_launch(ctx, d_b, n, d_ex, c, G, soft, d_acc,
+                                      cp ? d_cm_acc : nullptr, st, d_init);
         }
-        if (r != NCG_OK) return r;
-        // CM_acc in the reference's order: the terms added body by body.
-        if (cp && d_cm_acc) return ncg_cm_seq_launch(ctx, cterm, n, d_ex, 1, d_cm_acc, st);
-        return NCG_OK;
+        return r;
     }
     NCG_REQUIRE(prec == NCG_F64_FAST || prec == NCG_MIXED, "unknown precision %d", (int)prec);
     ncg_status r = ncg_tiled_order(ctx, d_b, n, d_ex, prec, st);
@@ -1013,11 +1006,9 @@ extern "C" ncg_status ncg_gravity_allpairs_static_dev(ncg_ctx *ctx, const ncg_bo
     // Every scratch word the kernels read is written first in the same call:
     // nothing needs clearing between calls.
     if (prec == NCG_F64_EXACT) {
-        ncg_status r = ncg_grav_exact_launch(ctx, db, n, d_exists, cp ? central : nullptr, G,
-                                             softening_parameter, d_acc, w.cterm, st, nullptr);
-        if (r != NCG_OK) return r;
-        if (want_cm) return ncg_cm_seq_launch(ctx, w.cterm, n, d_exists, 1, d_cm_acc, st);
-        return NCG_OK;
+        return ncg_grav_exact_launch(ctx, db, n, d_exists, cp ? central : nullptr, G,
+                                     softening_parameter, d_acc, want_cm ? d_cm_acc : nullptr,
+                                     st, nullptr);
     }
     if (!tiled)
         return ncg_small_launch(ctx, db, n, d_exists, cp ? central : nullptr, nullptr, G,
@@ -1065,10 +1056,9 @@ static ncg_status gravity_host(ncg_ctx *ctx, const ncg_body *bodies, int32_t n,
     DBody *db = dbuf<DBody>(ctx, "h_bodies", n);
     int32_t *dex = exists ? dbuf<int32_t>(ctx, "h_exists", n) : nullptr;
     double *dacc = dbuf<double>(ctx, "h_acc", 3 * (size_t)n);
-    double *dct = cp ? dbuf<double>(ctx, "h_cterm", 3 * (size_t)n) : nullptr;
     double *dcm = dbuf<double>(ctx, "h_cm", 4);
     double *dinit = start ? dbuf<double>(ctx, "h_start", 3 * (size_t)n) : nullptr;
-    if (!db || (exists && !dex) || !dacc || (cp && !dct) || !dcm || (start && !dinit))
+    if (!db || (exists && !dex) || !dacc || !dcm || (start && !dinit))
         return NCG_ERR_NOMEM;
     NCG_HIP(hipMemcpyAsync(db, bodies, sizeof(DBody) * (size_t)n, hipMemcpyHostToDevice, st));
     if (start)
@@ -1076,20 +1066,14 @@ static ncg_status gravity_host(ncg_ctx *ctx, const ncg_body *bodies, int32_t n,
                                st));
     if (exists)
         NCG_HIP(hipMemcpyAsync(dex, exists, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, st));
-    const bool exact = prec == NCG_F64_EXACT;
     ncg_status r = ncg_gravity_dev_impl(ctx, db, n, dex, central, G, softening_parameter, prec,
-                                        dacc, dct, (cp && !exact) ? dcm : nullptr, st, dinit);
+                                        dacc, nullptr, cp ? dcm : nullptr, st, dinit);
     if (r != NCG_OK) return r;
     // Holes keep the caller's values: copy back per existing body.
     double *hacc = hbuf<double>(ctx, "acc", 3 * (size_t)n);
     NCG_HIP(hipMemcpyAsync(hacc, dacc, sizeof(double) * 3 * (size_t)n, hipMemcpyDeviceToHost, st));
-    double *hct = nullptr;
-    if (cp && exact) {
-        hct = hbuf<double>(ctx, "cterm", 3 * (size_t)n);
-        NCG_HIP(hipMemcpyAsync(hct, dct, sizeof(double) * 3 * (size_t)n, hipMemcpyDeviceToHost, st));
-    }
     double hcm[4] = {0, 0, 0, 0};
-    if (cp && !exact) NCG_HIP(hipMemcpyAsync(hcm, dcm, sizeof(double) * 3, hipMemcpyDeviceToHost, st));
+    if (cp) NCG_HIP(hipMemcpyAsync(hcm, dcm, sizeof(double) * 3, hipMemcpyDeviceToHost, st));
     NCG_HIP(hipStreamSynchronize(st));
     for (int32_t k = 0; k < n; ++k) {
         if (exists && !exists[k]) continue;
@@ -1098,23 +1082,9 @@ static ncg_status gravity_host(ncg_ctx *ctx, const ncg_body *bodies, int32_t n,
         acc[3 * (size_t)k + 2] = hacc[3 * (size_t)k + 2];
     }
     if (cp && cm_acc) {
-        if (exact) {
-            // CM_acc accumulates body by body in index order (physics.c:80, 140-142).
-            double s0 = 0., s1 = 0., s2 = 0.;
-            for (int32_t k = 0; k < n; ++k) {
-                if (exists && !exists[k]) continue;
-                s0 += hct[3 * (size_t)k];
-                s1 += hct[3 * (size_t)k + 1];
-                s2 += hct[3 * (size_t)k + 2];
-            }
-            cm_acc[0] = s0;
-            cm_acc[1] = s1;
-            cm_acc[2] = s2;
-        } else {
-            cm_acc[0] = hcm[0];
-            cm_acc[1] = hcm[1];
-            cm_acc[2] = hcm[2];
-        }
+        cm_acc[0] = hcm[0];
+        cm_acc[1] = hcm[1];
+        cm_acc[2] = hcm[2];
     }
     return NCG_OK;
 }

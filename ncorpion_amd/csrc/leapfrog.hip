@@ -757,14 +757,13 @@ ncg_status leapfrog_run(ncg_ctx *ctx, ncg_body *d_bodies, int32_t n_in, int32_t 
     const bool use_graph = (flags & 1) != 0;
     const unsigned cap = ncg_replay_cap(ctx, 1u << 20);
     double *acc = dbuf<double>(ctx, "lf_acc", 3 * (size_t)ncap);
-    double *cterm = dbuf<double>(ctx, "lf_cterm", 3 * (size_t)ncap);
     double *cm = dbuf<double>(ctx, "lf_cm", 4);
     int2 *cand = dbuf<int2>(ctx, "lf_cand", cap);
     unsigned long long *cnt = dbuf<unsigned long long>(ctx, "lf_cnt", 1);
     unsigned char *dirty = dbuf<unsigned char>(ctx, "lf_dirty", (size_t)ncap + 4);
     unsigned *stat = dbuf<unsigned>(ctx, "lf_stat", 4);
     int *off = dbuf<int>(ctx, "lf_off", 2);
-    if (!acc || !cterm || !cm || !cand || !cnt || !dirty || !stat || !off) return NCG_ERR_NOMEM;
+    if (!acc || !cm || !cand || !cnt || !dirty || !stat || !off) return NCG_ERR_NOMEM;
     double present = 0.0;
     NCG_HIP(hipMemcpyAsync(&present, d_central + 7, sizeof(double), hipMemcpyDeviceToHost, st));
     NCG_HIP(hipStreamSynchronize(st));
@@ -783,8 +782,10 @@ ncg_status leapfrog_run(ncg_ctx *ctx, ncg_body *d_bodies, int32_t n_in, int32_t 
     NCG_CHECK_LAUNCH();
     const double G = grav_const, soft = softening;
 
-    auto collide = [&](double h) -> ncg_status {
-        hipLaunchKernelGGL(k_lf_zero_u64, dim3(1), dim3(1), 0, st, cnt);
+    // cleared: the candidate count is zero already (the exact field's launch
+    // clears it).
+    auto collide = [&](double h, bool cleared) -> ncg_status {
+        if (!cleared) hipLaunchKernelGGL(k_lf_zero_u64, dim3(1), dim3(1), 0, st, cnt);
         ncg_status r = ncg_candidates_launch(ctx, b, n, ex, h, cand, cap, cnt, st);
         if (r != NCG_OK) return r;
         if (n >= NCG_CP_MIN)
@@ -909,13 +910,13 @@ ncg_status leapfrog_run(ncg_ctx *ctx, ncg_body *d_bodies, int32_t n_in, int32_t 
     // A collision pass with dt h, checked: on a capacity error (or, under the
     // merger and fragmentation models, a resolved pair) the pass is undone
     // and replayed on the host.
-    auto collide_checked = [&](double h) -> ncg_status {
+    auto collide_checked = [&](double h, bool cleared) -> ncg_status {
         unsigned hs[3];
         ncg_status r = read_stat(hs);
         if (r != NCG_OK) return r;
         const unsigned before = hs[0];
         if ((r = copy_state(pass_b, pass_dc, nullptr, b, d_did_collide, nullptr, n)) != NCG_OK) return r;
-        if ((r = collide(h)) != NCG_OK) return r;
+        if ((r = collide(h, cleared)) != NCG_OK) return r;
         if ((r = read_stat(hs)) != NCG_OK) return r;
         if (hs[1] == 0u && !(model_host && hs[0] != before)) return NCG_OK;
         if ((r = copy_state(b, d_did_collide, nullptr, pass_b, pass_dc, nullptr, n)) != NCG_OK) return r;
@@ -1017,16 +1018,24 @@ ncg_status leapfrog_run(ncg_ctx *ctx, ncg_body *d_bodies, int32_t n_in, int32_t 
     cflag.present = cp ? 1 : 0;
     auto step = [&](bool checked) -> ncg_status {
         ncg_status r;
-        if (prec == NCG_F64_EXACT)
-            r = ncg_grav_exact_dev(ctx, b, n, ex, d_central, G, soft, acc, cterm, cp ? cm : nullptr, st);
+        // The exact field's launch forms CM_acc, kicks the bodies and the
+        // central body (which its other blocks do not read: positions and
+        // masses only) and clears the candidate count.
+        const bool fused = prec == NCG_F64_EXACT;
+        if (fused)
+            r = ncg_grav_exact_dev(ctx, b, n, ex, d_central, G, soft, acc, cm,
+                                   NcgKickTail{b, d_central, dt, cnt}, st);
         else
             r = ncg_tiled_eval(ctx, b, n, ex, cp ? &cflag : nullptr, cp ? d_central : nullptr, G,
                                soft, prec, acc, nullptr, cp ? cm : nullptr, st);
         if (r != NCG_OK) return r;
-        hipLaunchKernelGGL(k_lf_kick, dim3(g), dim3(LT), 0, st, (int)n, ex, dt, b, acc, d_central, cm);
-        NCG_CHECK_LAUNCH();
+        if (!fused) {
+            hipLaunchKernelGGL(k_lf_kick, dim3(g), dim3(LT), 0, st, (int)n, ex, dt, b, acc, d_central,
+                               cm);
+            NCG_CHECK_LAUNCH();
+        }
         if (coll) {
-            r = checked ? collide_checked(dt) : collide(dt);
+            r = checked ? collide_checked(dt, fused) : collide(dt, fused);
             if (r != NCG_OK) return r;
         }
         hipLaunchKernelGGL(k_lf_drift, dim3(g), dim3(LT), 0, st, (int)n, ex, dt, b, d_central);
@@ -1042,7 +1051,7 @@ ncg_status leapfrog_run(ncg_ctx *ctx, ncg_body *d_bodies, int32_t n_in, int32_t 
     if (flags & 2) {
         // rk4.c:871-879: brute_force and drift with dt / 2.
         if (coll) {
-            ncg_status r = collide_checked(0.5 * dt);
+            ncg_status r = collide_checked(0.5 * dt, false);
             if (r != NCG_OK) return r;
         }
         hipLaunchKernelGGL(k_lf_drift, dim3(g), dim3(LT), 0, st, (int)n, ex, 0.5 * dt, b, d_central);

@@ -145,11 +145,22 @@ ncg_status ncg_mesh_pass_dev_flags(ncg_ctx *ctx, ncg_body *d_bodies, int32_t n,
                                    int32_t one_collision_only, ncg_mesh_stats *stats,
                                    unsigned *flags, hipStream_t st);
 
+// What follows the exact field in the same launch (leapfrog): the velocities
+// of the existing bodies kb and of the central body kcen kicked by h
+// (rk4.c:68-107; with d_cm_acc only), and a counter cleared.  Nulls: nothing.
+struct NcgKickTail {
+    DBody *kb;
+    double *kcen;
+    double h;
+    unsigned long long *zero;
+};
+
 // Exact brute-force field with the central body in a device record (8
-// doubles {x, y, z, vx, vy, vz, M, present}); CM_acc summed in body order.
+// doubles {x, y, z, vx, vy, vz, M, present}); with d_cm_acc, CM_acc summed in
+// body order.
 ncg_status ncg_grav_exact_dev(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int32_t *d_ex,
                               const double *d_cen, double G, double soft, double *d_acc,
-                              double *d_cterm, double *d_cm_acc, hipStream_t st);
+                              double *d_cm_acc, const NcgKickTail &tail, hipStream_t st);
 
 // Candidates of brute_force's pass (collide_allpairs.hip), appended to
 // d_out[0 .. cap) with the count in *d_count (zeroed by the caller).
@@ -313,13 +324,10 @@ ncg_status ncg_small_launch(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int
                             const ncg_central *central, const double *d_central, double G,
                             double soft, double *d_acc, double *d_cterm, double *d_p3,
                             double *d_cm_acc, hipStream_t st);
-// Exact form (gravity_exact.hip): the field with per-body CM_acc terms d_cterm
-// (3n, written when the central body is present), and CM_acc summed from
-// them in body order.
+// Exact form (gravity_exact.hip): the field and, with d_cm_acc, CM_acc summed
+// in body order.
 // d_init (3n, or null): each body's sum starts from it instead of the
 // central term.
 ncg_status ncg_grav_exact_launch(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int32_t *d_ex,
                                  const ncg_central *c, double G, double soft, double *d_acc,
-                                 double *d_cterm, hipStream_t st, const double *d_init);
-ncg_status ncg_cm_seq_launch(ncg_ctx *ctx, const double *d_cterm, int32_t n, const int32_t *d_ex,
-                             int cp, double *d_cm_acc, hipStream_t st);
+                                 double *d_cm_acc, hipStream_t st, const double *d_init);

@@ -210,3 +210,43 @@ def test_start_values_equal_central_term(ctx, n, prec):
     else:
         tol = 1e-12 if prec == "fast64" else 1e-6
         assert rel_err(got[live], ref[live])[0] < tol
+
+
+def _exact_edge_bodies(n, kind):
+    rng = np.random.default_rng(n + len(kind))
+    b = np.zeros((n, 8))
+    b[:, 0:3] = rng.normal(size=(n, 3))
+    b[:, 6] = rng.uniform(1e-9, 1e-8, n)
+    b[:, 7] = rng.uniform(1e-4, 1e-3, n)
+    if kind == "planar":          # zero separations on an axis, of both signs of zero
+        b[:, 2] = 0.0
+        b[::3, 2] = -0.0
+        b[1::2, 1] = 0.25
+    elif kind == "window":        # every check of the window form fails somewhere
+        b[0, 0] = 1e-60           # a coordinate below 2^-140
+        b[n // 2, 6] = 1e-40      # G m below 2^-100
+        b[n // 3, 6] = -1e-9      # negative
+        b[n // 4, 0:3] *= 1e40    # r2 above 2^190
+        b[n - 1, 6] = 0.0
+        b[n - 2, 0:3] = b[n - 3, 0:3] + 1e-35  # r2 far below 1
+    return b
+
+
+# Edges of the workgroup-per-4-bodies form (chunks of 192 bodies, wavefronts of
+# 64) and operands outside the window of the branch-free quotients.
+@pytest.mark.parametrize("soft", [0.0, 1e-3])
+@pytest.mark.parametrize("n,kind", [(4, ""), (5, "planar"), (63, "planar"), (64, ""), (65, "window"),
+                                    (191, "window"), (192, "planar"), (193, "window"),
+                                    (577, "planar"), (1153, "window")])
+def test_exact_bitwise_edges(ctx, n, kind, soft):
+    b = _exact_edge_bodies(n, kind)
+    ex = (np.random.default_rng(n).uniform(size=n) > 0.1).astype(np.int32)
+    cen = (0.1, 0.2, -0.3, 1.0)
+    for e in (None, ex):
+        ref, rcm = orc.vector_field_brute(b, e, cen, 1.0, soft)
+        acc, cm = ctx.gravity_allpairs(b, e, cen, 1.0, soft, "exact")
+        on = slice(None) if e is None else e != 0
+        # Coincident bodies give NaN in both; its sign is the processor's.
+        a, r = acc[on], ref[on]
+        assert np.all((bits(a) == bits(r)) | (np.isnan(a) & np.isnan(r)))
+        assert np.array_equal(bits(cm), bits(rcm))
