@@ -21,7 +21,10 @@
 //   Kbar_s = h w_s / 6 * ybar',  for s = 4..1:
 //     Ybar_s = (VJP_x(a at X_s; Kbar_s.v), Kbar_s.x);  ybar += Ybar_s;
 //     Kbar_{s-1} += c_s h Ybar_s                     (c = 1/2, 1/2, 1)
+#include <algorithm>
+
 #include "ncg_internal.hpp"
+#include "sym_dev.hpp"
 
 namespace {
 
@@ -131,6 +134,155 @@ __global__ __launch_bounds__(AT) void k_vjp_reduce(const double4 *__restrict__ p
     gx[3 * (size_t)i + 1] = G * t.y;
     gx[3 * (size_t)i + 2] = G * t.z;
     gm[i] = G * t.w;
+}
+
+// The pair part by unordered pairs (sym_dev.hpp): with u = m_i lam_j - m_j
+// lam_i, the pair adds T u to g_x_i and -T u to g_x_j, -G lam_j . d / D^3 to
+// g_m_i and G lam_i . d / D^3 to g_m_j: 47 FP64 instructions and one v_rsq_f64 a
+// pair, against 38 and one for each of the two.  16,384 bodies: 276 us (382 by
+// ordered pairs); four bodies i a wavefront spilled (1320 us), with fewer
+// wavefronts a SIMD 384.
+constexpr int VI = 2;    // bodies i of a wavefront
+constexpr int VROW = SY_WAVES * VI;
+
+struct VjpRec {
+    double x, y, z, m, lx, ly, lz, s;
+};
+
+template <bool DIAG>
+__device__ inline void vjp_block(const VjpRec *ri, int i0, int j, const VjpRec &q, double (*acc)[VI],
+                                 double *bj)
+{
+#pragma unroll
+    for (int u = 0; u < VI; ++u) {
+        const VjpRec &a = ri[u];
+        const double dx = q.x - a.x, dy = q.y - a.y, dz = q.z - a.z;
+        const double e = a.s + q.s;
+        const double D2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, e * e)));
+        double y = __builtin_amdgcn_rsq(D2);
+        y = y * fma(-0.5 * D2, y * y, 1.5);
+        const double y2 = y * y;
+        double i3 = y2 * y, i5 = i3 * y2;
+        if (DIAG) {
+            i3 = j <= i0 + u ? 0.0 : i3;
+            i5 = j <= i0 + u ? 0.0 : i5;
+        }
+        const double ux = fma(a.m, q.lx, -q.m * a.lx);
+        const double uy = fma(a.m, q.ly, -q.m * a.ly);
+        const double uz = fma(a.m, q.lz, -q.m * a.lz);
+        const double du3 = 3.0 * fma(dx, ux, fma(dy, uy, dz * uz)) * i5;
+        const double tx = fma(ux, i3, -dx * du3), ty = fma(uy, i3, -dy * du3),
+                     tz = fma(uz, i3, -dz * du3);
+        acc[0][u] += tx;
+        acc[1][u] += ty;
+        acc[2][u] += tz;
+        bj[0] -= tx;
+        bj[1] -= ty;
+        bj[2] -= tz;
+        acc[3][u] = fma(-fma(q.lx, dx, fma(q.ly, dy, q.lz * dz)), i3, acc[3][u]);
+        bj[3] = fma(fma(a.lx, dx, fma(a.ly, dy, a.lz * dz)), i3, bj[3]);
+    }
+}
+
+__global__ __launch_bounds__(SY_T, 4) void k_vjp_sym(const VjpRec *__restrict__ jv, SymShape S,
+                                                     double *__restrict__ pi,
+                                                     double *__restrict__ pj)
+{
+    __shared__ double rec[8][SY_T];
+    __shared__ double js[4][SY_T];
+    int r, c;
+    sym_place(S, blockIdx.x, r, c);
+    const int n = S.n, tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j0 = c * SY_T, row0 = r * S.W;
+    {
+        VjpRec q = jv[min(j0 + tid, n - 1)];
+        // A slot past n: far from every body, without mass or cotangent.
+        if (j0 + tid >= n) q = VjpRec{1e100, 1e100, 1e100, 0., 0., 0., 0., 0.};
+        rec[0][tid] = q.x;
+        rec[1][tid] = q.y;
+        rec[2][tid] = q.z;
+        rec[3][tid] = q.m;
+        rec[4][tid] = q.lx;
+        rec[5][tid] = q.ly;
+        rec[6][tid] = q.lz;
+        rec[7][tid] = q.s;
+        for (int d = 0; d < 4; ++d) js[d][tid] = 0.0;
+    }
+    __syncthreads();
+    for (int row = row0; row < row0 + S.W; row += VROW) {
+        if (row >= n || row >= j0 + SY_T) break;
+        const int i0 = row + w * VI;
+        VjpRec ri[VI];
+#pragma unroll
+        for (int u = 0; u < VI; ++u) {
+            ri[u] = jv[min(i0 + u, n - 1)];  // uniform address: scalar loads
+            if (i0 + u >= n) ri[u].m = ri[u].lx = ri[u].ly = ri[u].lz = 0.0;
+        }
+        double acc[4][VI];
+#pragma unroll
+        for (int u = 0; u < VI; ++u) acc[0][u] = acc[1][u] = acc[2][u] = acc[3][u] = 0.0;
+        for (int s = 0; s < SY_WAVES; ++s) {
+            const int kb = ((w + s) & (SY_WAVES - 1)) * 64, k = kb + lane, jb = j0 + kb;
+            if (jb + 63 > i0) {
+                const VjpRec q{rec[0][k], rec[1][k], rec[2][k], rec[3][k],
+                               rec[4][k], rec[5][k], rec[6][k], rec[7][k]};
+                double bj[4] = {js[0][k], js[1][k], js[2][k], js[3][k]};
+                if (jb >= i0 + VI) vjp_block<false>(ri, i0, jb + lane, q, acc, bj);
+                else vjp_block<true>(ri, i0, jb + lane, q, acc, bj);
+                for (int d = 0; d < 4; ++d) js[d][k] = bj[d];
+            }
+            __syncthreads();
+        }
+        double v[4 * VI];  // value 4 u + d: a lane ends with the sums of one body
+#pragma unroll
+        for (int u = 0; u < VI; ++u)
+            for (int d = 0; d < 4; ++d) v[4 * u + d] = acc[d][u];
+        const int h = lanes_sum4<VI>(v, lane);  // components 2 h, 2 h + 1
+        const int u = h >> 1;
+        if ((lane & ~12) == 0 && i0 + u < n) {
+            double *o = pi + 4 * (S.ioff(c) + i0 + u) + 2 * (h & 1);
+            o[0] = v[0];
+            o[1] = v[1];
+        }
+    }
+    if (j0 + tid >= row0) {
+        double *o = pj + 4 * (S.joff(r) + (j0 - row0) + tid);
+        for (int d = 0; d < 4; ++d) o[d] = js[d][tid];
+    }
+}
+
+// Sums of VS bodies' components over chunks and row groups in a fixed order,
+// times G: 16 interleaved shares each (one share a component took 28 us at
+// 16,384 bodies, bound by the reads' latency).
+constexpr int VS = 16, VQ = 16;
+
+__global__ __launch_bounds__(AT) void k_vjp_sym_sum(SymShape S, const double *__restrict__ pi,
+                                                    const double *__restrict__ pj, double G,
+                                                    double *__restrict__ gx,
+                                                    double *__restrict__ gm)
+{
+    __shared__ double sh[VQ][4 * VS];
+    const int s0 = blockIdx.x * VS;
+    for (int item = threadIdx.x; item < VQ * 4 * VS; item += AT) {
+        const int q = item / (4 * VS), e = item % (4 * VS), s = s0 + e / 4;
+        double a = 0.0;
+        if (s < S.n) {
+            a = share_sum<VQ>(s / S.C + q, S.chunks,
+                              [&](int c) { return pi[4 * (S.ioff(c) + s0) + e]; });
+            a += share_sum<VQ>(q, s / S.W + 1, [&](int r) {
+                return pj[4 * (S.joff(r) + s0 - (long)r * S.W) + e];
+            });
+        }
+        sh[q][e] = a;
+    }
+    __syncthreads();
+    const int e = threadIdx.x, s = s0 + e / 4, d = e & 3;
+    if (e >= 4 * VS || s >= S.n) return;
+    double a = 0.0;
+    for (int q = 0; q < VQ; ++q) a += sh[q][e];
+    if (d < 3) gx[3 * (size_t)s + d] = G * a;
+    else gm[s] = G * a;
 }
 
 // Central part, added to g_x / g_m; per-block partials of g_C (3) and g_M.
@@ -307,6 +459,12 @@ __global__ void k_add(double *__restrict__ a, const double *__restrict__ b, int 
 
 }  // namespace
 
+// Bodies for which the pair part runs by unordered pairs: 114 us against 112 by
+// ordered ones at 8192 bodies (too few workgroups), 57 against 37 at 4096, 364
+// against 438 at 16,384 with the sums; above 131,072 the partial sums take more
+// than 4 GB.
+static constexpr int VJP_SYM_MIN = 10240, VJP_SYM_MAX = 131072;
+
 // VJP at body state b (positions and masses) with central state cen (8):
 // gx (3n) =; gm (n) += when acc_gm else =; gcm (4: g_C, g_M) =.
 static ncg_status vjp_impl(ncg_ctx *ctx, const DBody *b, int32_t n, const double *cen, double G,
@@ -324,15 +482,29 @@ static ncg_status vjp_impl(ncg_ctx *ctx, const DBody *b, int32_t n, const double
     nsplit = (int)cdiv(n, per);
     double *part = dbuf<double>(ctx, "v_part", 4 * (size_t)nb);
     double *jv = dbuf<double>(ctx, "v_jv", 8 * (size_t)n);
-    double4 *pp = dbuf<double4>(ctx, "v_pp", (size_t)nsplit * n);
-    if (!gm_tmp || !part || !jv || !pp) return NCG_ERR_NOMEM;
+    if (!gm_tmp || !part || !jv) return NCG_ERR_NOMEM;
     hipLaunchKernelGGL(k_vjp_pack, dim3(nb), dim3(AT), 0, st, b, (int)n, lam, soft, jv);
-    {
+    if (n >= VJP_SYM_MIN && n <= VJP_SYM_MAX) {
+        const SymShape S = sym_shape(n, 1, VI, n <= 32768 ? 4 : 8);
+        double *pi = dbuf<double>(ctx, "v_pi", 4 * (size_t)S.islots());
+        double *pj = dbuf<double>(ctx, "v_pj", 4 * (size_t)S.jslots());
+        if (!pi || !pj) return NCG_ERR_NOMEM;
         ProfScope ps(ctx, st, "vjp");
-        hipLaunchKernelGGL(k_vjp_pairs, dim3(nb, nsplit), dim3(AT), 0, st, jv, (int)n, per, pp);
+        hipLaunchKernelGGL(k_vjp_sym, dim3((unsigned)S.workgroups()), dim3(SY_T), 0, st,
+                           reinterpret_cast<const VjpRec *>(jv), S, pi, pj);
+        hipLaunchKernelGGL(k_vjp_sym_sum, dim3(cdiv(n, VS)), dim3(AT), 0, st, S, pi, pj, G, gx,
+                           gm_tmp);
         NCG_CHECK_LAUNCH();
+    } else {
+        double4 *pp = dbuf<double4>(ctx, "v_pp", (size_t)nsplit * n);
+        if (!pp) return NCG_ERR_NOMEM;
+        {
+            ProfScope ps(ctx, st, "vjp");
+            hipLaunchKernelGGL(k_vjp_pairs, dim3(nb, nsplit), dim3(AT), 0, st, jv, (int)n, per, pp);
+            NCG_CHECK_LAUNCH();
+        }
+        hipLaunchKernelGGL(k_vjp_reduce, dim3(nb), dim3(AT), 0, st, pp, nsplit, (int)n, G, gx, gm_tmp);
     }
-    hipLaunchKernelGGL(k_vjp_reduce, dim3(nb), dim3(AT), 0, st, pp, nsplit, (int)n, G, gx, gm_tmp);
     hipLaunchKernelGGL(k_vjp_central, dim3(nb), dim3(AT), 0, st, b, (int)n, cen, lam, lamc, G, gx,
                        gm_tmp, part);
     hipLaunchKernelGGL(k_sum4, dim3(1), dim3(AT), 0, st, part, nb, gcm, 0);

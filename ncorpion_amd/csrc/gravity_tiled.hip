@@ -738,10 +738,21 @@ static ncg_status tiled_order_w(ncg_ctx *ctx, const TiledShape &t, const TiledWo
     return NCG_OK;
 }
 
+// Whether the FP64-fast form runs by unordered pairs (gravity_sym.hip): with a
+// launch shape of the caller's (ncg_set_tiling) the split kernel runs in that
+// shape, and above NCG_SYM_MAX bodies the partial sums of the unordered form
+// would take more than 3.3 GB.  Faster at every size between (calls of 4200
+// bodies 46 us against 112, 50,021 1.35 ms against 1.87, 200,000 17.8 against 24).
+static bool sym_form(const ncg_ctx *ctx, int32_t n, ncg_precision prec)
+{
+    return prec == NCG_F64_FAST && n > SMALL_N && n <= NCG_SYM_MAX && !ctx->tiled_explicit;
+}
+
 ncg_status ncg_tiled_order(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int32_t *d_ex,
                            ncg_precision prec, hipStream_t st)
 {
     if (n <= SMALL_N) return NCG_OK;  // the direct form needs no order
+    if (sym_form(ctx, n, prec) && !d_ex) return NCG_OK;  // body order
     const TiledShape t = tiled_shape(ctx, n, NCG_MIXED);
     TiledWork w;
     ncg_status r = work_order_ctx(ctx, t, n, st, w);
@@ -846,6 +857,16 @@ ncg_status ncg_tiled_eval(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int32
         ProfScope ps(ctx, st, prec == NCG_F64_FAST ? "pairs_fast64" : "pairs_mixed");
         return ncg_small_launch(ctx, d_b, n, d_ex, c, d_central, G, soft, d_acc, cterm, p3,
                                 d_cm_acc, st);
+    }
+    if (sym_form(ctx, n, prec)) {
+        const int *perm = nullptr, *nvalid = nullptr;
+        if (d_ex) {  // the order of ncg_tiled_order: existing bodies first
+            perm = dbuf<int>(ctx, "t_perm", n);
+            Scal *sc = dbuf<Scal>(ctx, "t_scal", 1);
+            if (!perm || !sc) return NCG_ERR_NOMEM;
+            nvalid = &sc->nvalid;
+        }
+        return ncg_gravity_sym(ctx, d_b, n, perm, nvalid, c, d_central, G, soft, d_acc, d_cm_acc, st);
     }
     const TiledShape t = tiled_shape(ctx, n, prec);
     TiledWork w;

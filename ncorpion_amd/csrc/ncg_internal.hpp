@@ -316,6 +316,13 @@ ncg_status ncg_gravity_dev_impl(ncg_ctx *ctx, const DBody *d_bodies, int32_t n,
                                 double soft, ncg_precision prec, double *d_acc,
                                 double *d_cterm, double *d_cm_acc, hipStream_t s,
                                 const double *d_init = nullptr);
+// FP64-fast form by unordered pairs (gravity_sym.hip), in slot order: d_perm
+// (slots to bodies; null: body order) and d_nvalid (existing bodies; null: n).
+// d_central: the central body in a device record; else c (may be null).
+constexpr int NCG_SYM_MAX = 262144;
+ncg_status ncg_gravity_sym(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int *d_perm,
+                           const int *d_nvalid, const ncg_central *c, const double *d_central,
+                           double G, double soft, double *d_acc, double *d_cm_acc, hipStream_t st);
 // Direct form of the fast gravity forms for 1..4096 bodies (k_small): one
 // wavefront per body; with d_cm_acc, CM_acc as a fixed-shape tree sum of the
 // terms d_cterm (3n) through d_p3 (3 * ncg_small_partials(n) doubles).

@@ -250,3 +250,46 @@ def test_exact_bitwise_edges(ctx, n, kind, soft):
         a, r = acc[on], ref[on]
         assert np.all((bits(a) == bits(r)) | (np.isnan(a) & np.isnan(r)))
         assert np.array_equal(bits(cm), bits(rcm))
+
+
+# The FP64-fast form by unordered pairs: chunks of 1024 bodies, row groups of 64
+# to 512 (more rows a group above 20,000 and 65,536 bodies), remainders of every
+# kind, holes at the ends; both softening kernels; the split kernel in a shape of
+# the caller's gives the same to rounding (~sqrt(n) ulps of the sum; 1e-13).
+@pytest.mark.parametrize("n,soft", [(4097, 0.0), (5120, 0.5), (8191, 0.0), (20001, 0.5),
+                                    (65537, 0.0)])
+def test_fast64_pairs_match_split_form(n, soft):
+    import torch
+    from ncorpion_amd import Context
+    m, R = ic.disk_c3_masses(n, n)
+    b = ic.disk(n, seed=n, masses=m, radii=R)
+    ex = (np.random.default_rng(n).uniform(size=n) > 0.07).astype(np.int32)
+    ex[[0, -1]] = 0
+    cen = (1e-3, 2e-3, -1e-3, 1.0)
+    bt, et = torch.from_numpy(b).cuda(), torch.from_numpy(ex).cuda()
+    got = {}
+    for shape in (None, (1, 32)):
+        ctx = Context(0)
+        try:
+            if shape:
+                ctx.set_tiling(shape[0], shape[1], 0.35, 0)
+            for e in (None, et):
+                acc = torch.full((n, 3), 7.0, dtype=torch.float64, device="cuda")
+                cm = torch.zeros(3, dtype=torch.float64, device="cuda")
+                torch.cuda.synchronize()
+                ctx.gravity_allpairs_dev(bt, acc, e, cen, 1.0, soft, "fast64", cm)
+                ctx.synchronize()
+                got[shape is None, e is None] = (acc.cpu().numpy(), cm.cpu().numpy())
+        finally:
+            ctx.close()
+    for whole in (True, False):
+        (a, ca), (r, cr) = got[True, whole], got[False, whole]
+        on = slice(None) if whole else ex != 0
+        if not whole:
+            assert np.all(a[ex == 0] == 7.0)
+        assert rel_err(a[on], r[on])[1] < 1e-13
+        assert np.abs(ca - cr).max() < 1e-13 * np.abs(m).sum()
+    rows = np.array([1, n // 2, n - 2])
+    ref = orc.vector_field_rows(b, rows, None, cen, 1.0, soft)
+    ref = ref[0] if isinstance(ref, tuple) else ref
+    assert rel_err(got[True, True][0][rows], ref)[0] < 1e-12
