@@ -161,6 +161,8 @@ __global__ __launch_bounds__(FT) void k_sym_finish(const DBody *__restrict__ b,
                                                    const double *__restrict__ pj, int cp, double cx,
                                                    double cy, double cz, double mu,
                                                    const double *__restrict__ dcen, double G,
+                                                   const double *__restrict__ near, int nnear,
+                                                   const Scal *__restrict__ scal,
                                                    double *__restrict__ acc,
                                                    double *__restrict__ cmpart)
 {
@@ -176,6 +178,8 @@ __global__ __launch_bounds__(FT) void k_sym_finish(const DBody *__restrict__ b,
             a = share_sum<FQ>(s / SY_C + q, c1, [&](int c) { return pi[3 * (S.ioff(c) + s0) + e]; });
             a += share_sum<FQ>(q, r1,
                            [&](int r) { return pj[3 * (S.joff(r) + s0 - (long)r * S.W) + e]; });
+            // The mixed form's near terms.
+            if (q < nnear) a += near[3 * ((size_t)q * S.n + s0) + e];
         }
         sh[q][e] = a;
     }
@@ -197,6 +201,10 @@ __global__ __launch_bounds__(FT) void k_sym_finish(const DBody *__restrict__ b,
             const int e = 3 * tid + d;
             a[d] = 0.0;
             for (int q = 0; q < FQ; ++q) a[d] += sh[q][e];
+        }
+        if (scal) {  // the mixed form's powers of two
+            const int ex = mass_exp(*scal, G) - 2 * scal->lexp;
+            for (int d = 0; d < 3; ++d) a[d] = ldexp(a[d], ex);
         }
         if (cp) {
             const DBody q = b[k];
@@ -231,6 +239,319 @@ __global__ __launch_bounds__(FT) void k_sym_records(const DBody *__restrict__ b,
     const DBody q = b[perm ? perm[s] : s];
     jd[s] = make_double4(q.x, q.y, q.z, G * q.mass);
     jsig[s] = soft * q.radius;
+}
+
+// ---- mixed form ---------------------------------------------------------------
+// The bodies are in Hilbert order, cut into groups of 64.  For two groups a
+// decision from their boxes (near_pair, one bit, the same for both orders)
+// picks the form of their pairs:
+//   near: FP64, ordered, by k_mix_near;
+//   far:  FP32, unordered, by k_pairs_mix: separations d = W_j - v_i of positions
+//         taken from the box centre of i's group in FP64 and rounded once; 16
+//         instructions and a v_rsq_f32 a pair, where the scaled far term of the
+//         split kernel takes 11 and one for each of the two: 51 against 76
+//         clocks of issue a wavefront, of which 73 are reached (the rest: j
+//         records and sums in LDS, barriers).  Operands are vector registers (a
+//         scalar one takes the issue from 2.6 to 4.4 clocks).
+// A lane's FP32 sums are 16 terms of a body j, or 16 of a body i, and i's over 8
+// lanes; all after that are FP64.  Positions and G m are scaled by powers of two
+// (the box's edge and the largest G m about 1), so that no system of units over-
+// or underflows FP32 (the FP64 terms are unchanged by it, but for results at the
+// ends of its range).
+// Calls of 262,144 bodies: 19.2 ms with the split kernel, 16.1 here; 100,003:
+// 3.40 and 2.87; 32,800: 0.57 and 0.50; the field's error against FP64 is that
+// of the split kernel (4.9e-9 and 5.0e-9, 2.3e-9 and 2.2e-9, 1.8e-9 and 1.3e-9).
+// Eight bodies i a wavefront: 21.2 ms at 262,144 (the j records and sums come
+// twice as often); sums over all lanes in FP32: error +10 %.
+constexpr int MI = 16;            // bodies i of a wavefront
+constexpr int MG = 64;            // bodies of a group: half a row of wavefronts
+constexpr int MNEAR = 4;          // partial sums of a body's near terms
+constexpr int NW = 8;             // wavefronts that form one
+constexpr int MROW = SY_WAVES * MI;
+static_assert(MROW == 2 * MG, "a row of wavefronts is two groups");
+
+__global__ __launch_bounds__(64) void k_mix_records(const DBody *__restrict__ b,
+                                                    const int *__restrict__ perm,
+                                                    const Scal *__restrict__ scal, double G,
+                                                    double soft, double4 *__restrict__ jd,
+                                                    double *__restrict__ jsig,
+                                                    TileHdr *__restrict__ hdr)
+{
+    const Scal S = *scal;
+    const int g = blockIdx.x, lane = threadIdx.x, s = g * MG + lane;
+    if (g * MG >= S.nvalid) return;
+    const DBody q = b[perm[min(s, S.nvalid - 1)]];
+    const double gm = G * q.mass;
+    const double p[3] = {ldexp(q.x, -S.lexp), ldexp(q.y, -S.lexp), ldexp(q.z, -S.lexp)};
+    const double sg = ldexp(gm, -mass_exp(S, G));
+    // Slots past the last body repeat it without mass.
+    jd[s] = make_double4(p[0], p[1], p[2], s < S.nvalid ? sg : 0.0);
+    jsig[s] = ldexp(soft * q.radius, -S.lexp);
+    // Negative, not finite, or a term of it could leave FP32's normal range
+    // (near_pair bounds the distances).
+    const bool bad = __any(!(sg == 0.0 || (sg >= 0x1p-96 && sg <= 2.0)));
+    double A[3];
+    float H[3];
+    for (int c = 0; c < 3; ++c) {
+        double lo = p[c], hi = p[c];
+        for (int o = 32; o > 0; o >>= 1) {
+            lo = fmin(lo, __shfl_xor(lo, o));
+            hi = fmax(hi, __shfl_xor(hi, o));
+        }
+        A[c] = 0.5 * (lo + hi);
+        const double h = fmax(hi - A[c], A[c] - lo);
+        H[c] = (float)h;
+        if ((double)H[c] < h) H[c] = nextafterf(H[c], 3.0e38f);
+    }
+    if (lane == 0) {
+        TileHdr th;
+        th.ax = A[0];
+        th.ay = A[1];
+        th.az = A[2];
+        th.hx = H[0];
+        th.hy = H[1];
+        th.hz = H[2];
+        th.count = 0;
+        th.smax = bad ? INFINITY : 0.f;
+        th.smin = 0.f;
+        hdr[g] = th;
+    }
+}
+
+// Near unless the box distance is at least theta times (anchor distance + half
+// extents), beyond FP32 resolution of the largest softening length, and the
+// distances are in the range that FP32 terms are safe in (scaled units; bodies
+// may have left the box that set the scale); a group with an unfit G m (smax
+// set) is near to all, as is any whose box is NaN.
+__device__ inline bool near_pair(const TileHdr &a, const TileHdr &b, double theta, double eps2x)
+{
+    const double Cx = fabs(a.ax - b.ax), Cy = fabs(a.ay - b.ay), Cz = fabs(a.az - b.az);
+    const double gx = fmax(0.0, Cx - ((double)a.hx + b.hx));
+    const double gy = fmax(0.0, Cy - ((double)a.hy + b.hy));
+    const double gz = fmax(0.0, Cz - ((double)a.hz + b.hz));
+    const double dmin2 = gx * gx + gy * gy + gz * gz;
+    const double ha = sqrt((double)a.hx * a.hx + (double)a.hy * a.hy + (double)a.hz * a.hz);
+    const double hb = sqrt((double)b.hx * b.hx + (double)b.hy * b.hy + (double)b.hz * b.hz);
+    const double size = sqrt(Cx * Cx + Cy * Cy + Cz * Cz) + (ha + hb);
+    const bool far = dmin2 >= theta * theta * size * size && dmin2 > eps2x && dmin2 >= 0x1p-50 &&
+                     size <= 0x1p4 && a.smax == 0.f && b.smax == 0.f;
+    return !far;
+}
+
+// Bit h of group g's row: g and h are far.
+__global__ __launch_bounds__(64) void k_mix_mask(const TileHdr *__restrict__ hdr,
+                                                 const Scal *__restrict__ scal, int nw, double theta,
+                                                 double soft, unsigned long long *__restrict__ mask)
+{
+    const int ng = (scal->nvalid + MG - 1) / MG;
+    const int g = blockIdx.x, h = blockIdx.y * 64 + (int)threadIdx.x;
+    bool far = false;
+    if (g < ng && h < ng) {
+        // In this order for both bits of the pair, which must be one.
+        const TileHdr a = hdr[min(g, h)], b = hdr[max(g, h)];
+        const double eps = ldexp(2.0 * soft * scal->rmax, -scal->lexp);
+        far = !near_pair(a, b, theta, eps * eps * 67108864.0 /* 2^26 */);
+    }
+    const unsigned long long bits = __ballot(far);
+    if (threadIdx.x == 0) mask[(size_t)g * nw + blockIdx.y] = bits;
+}
+
+// Near terms: body i per lane, the near groups h = share modulo MNEAR NW with
+// wave-uniform addresses.  FP64 issue; 32 shares, because a few groups (the
+// sparse rim of a disk) are near to most others and last: with 8 shares the
+// kernel took 2.32 ms at 262,144 bodies and 0.98 at 65,536, with 32 1.29 and 0.28.
+constexpr unsigned long long near_step(int shares)
+{
+    unsigned long long v = 0;
+    for (int k = 0; k < 64; k += shares) v |= 1ull << k;
+    return v;
+}
+constexpr unsigned long long NEAR_STEP = near_step(MNEAR * NW);
+
+template <bool SOFT>
+__global__ __launch_bounds__(64 * NW) void k_mix_near(const double4 *__restrict__ jd,
+                                                 const double *__restrict__ jsig,
+                                                 const Scal *__restrict__ scal, int nw, int nslots,
+                                                 const unsigned long long *__restrict__ mask,
+                                                 double *__restrict__ part)
+{
+    __shared__ double sum[NW][3][MG];
+    const int nv = scal->nvalid, ng = (nv + MG - 1) / MG;
+    const int g = blockIdx.x, lane = threadIdx.x & 63, i = g * MG + lane;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int share = blockIdx.y * NW + wv;
+    if (g >= ng) return;
+    const double4 me = jd[i];
+    const double si = SOFT ? jsig[i] : 0.0;
+    double ax = 0.0, ay = 0.0, az = 0.0;
+    const unsigned long long *row = mask + (size_t)g * nw;
+    for (int w = 0; w * 64 < ng; ++w) {
+        unsigned long long bits = ~row[w] & (NEAR_STEP << share);
+        if (w * 64 + 64 > ng) bits &= ~0ull >> (w * 64 + 64 - ng);
+        while (bits) {
+            const int h = w * 64 + __ffsll((long long)bits) - 1;
+            bits &= bits - 1;
+            const int jb = h * MG, cnt = min(MG, nv - jb);
+            if (h == g) {
+                for (int jj = 0; jj < cnt; ++jj)
+                    near_term_self<1, SOFT>(jd[jb + jj], SOFT ? jsig[jb + jj] : 0.0, jb + jj, i, MG,
+                                            &me.x, &me.y, &me.z, &si, &ax, &ay, &az);
+            } else if (cnt == MG) {
+#pragma unroll 4
+                for (int jj = 0; jj < MG; ++jj)
+                    near_term<1, SOFT>(jd[jb + jj], SOFT ? jsig[jb + jj] : 0.0, &me.x, &me.y, &me.z,
+                                       &si, &ax, &ay, &az);
+            } else {
+                for (int jj = 0; jj < cnt; ++jj)
+                    near_term<1, SOFT>(jd[jb + jj], SOFT ? jsig[jb + jj] : 0.0, &me.x, &me.y, &me.z,
+                                       &si, &ax, &ay, &az);
+            }
+        }
+    }
+    sum[wv][0][lane] = ax;
+    sum[wv][1][lane] = ay;
+    sum[wv][2][lane] = az;
+    __syncthreads();
+    for (int e = threadIdx.x; e < 3 * MG; e += 64 * NW) {
+        const int s = e / 3, d = e - 3 * s;
+        double v = 0.0;
+        for (int q = 0; q < NW; ++q) v += sum[q][d][s];
+        if (g * MG + s < nv) part[3 * ((size_t)blockIdx.y * nslots + g * MG) + e] = v;
+    }
+}
+
+template <int CTRL>
+__device__ inline float dpp_get32(float v)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+
+template <int N, int CTRL>
+__device__ inline void halve32(float *a, bool up)
+{
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        const float keep = up ? a[q + N] : a[q], give = up ? a[q] : a[q + N];
+        a[q] = keep + dpp_get32<CTRL>(give);
+    }
+}
+
+// One workgroup per (row group r, chunk c) with pairs j > i, as k_pairs_sym.
+__global__ __launch_bounds__(SY_T, 4) void k_pairs_mix(const double4 *__restrict__ jd,
+                                                       const TileHdr *__restrict__ hdr,
+                                                       const Scal *__restrict__ scal, int nw,
+                                                       const unsigned long long *__restrict__ mask,
+                                                       SymShape S, double *__restrict__ pi,
+                                                       double *__restrict__ pj)
+{
+    __shared__ double4 rec[SY_C];
+    __shared__ double js[3][SY_C];
+    int r, c;
+    sym_place(S, blockIdx.x, r, c);
+    const int nv = scal->nvalid, tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j0 = c * SY_C, row0 = r * S.W, h0 = j0 / MG;
+    if (j0 >= nv || row0 >= nv) return;
+#pragma unroll
+    for (int h = 0; h < SY_NB; ++h) {
+        const int k = h * SY_T + tid;
+        // Slots up to the end of the last group hold records.
+        rec[k] = jd[min(j0 + k, (nv + MG - 1) / MG * MG - 1)];
+        js[0][k] = js[1][k] = js[2][k] = 0.0;
+    }
+    __syncthreads();
+    const int ng = (nv + MG - 1) / MG;
+    for (int row = row0; row < row0 + S.W; row += MROW) {
+        if (row >= nv || row >= j0 + SY_C) break;
+        const int i0 = row + w * MI, g = min(i0 / MG, ng - 1);
+        // The chunk's groups (a power of two of them, within one word) that are
+        // far from g and above it.
+        unsigned bits = 0, any = 0;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int f = row / MG + e;
+            if (f >= ng) continue;
+            unsigned v = (unsigned)(mask[(size_t)f * nw + (h0 >> 6)] >> (h0 & 63)) &
+                         ((1u << (SY_C / MG)) - 1u);
+            if (f >= h0) v &= ~((2u << (f - h0)) - 1u);
+            any |= v;
+            if (f == i0 / MG) bits = v;
+        }
+        double sum[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+        float acc[3 * MI];
+#pragma unroll
+        for (int q = 0; q < 3 * MI; ++q) acc[q] = 0.f;
+        if (any) {  // uniform in the workgroup
+            const TileHdr th = hdr[g];
+            float vx[MI], vy[MI], vz[MI], mi[MI];
+#pragma unroll
+            for (int u = 0; u < MI; ++u) {
+                const double4 p = jd[min(i0 + u, ng * MG - 1)];
+                vx[u] = (float)(p.x - th.ax);
+                vy[u] = (float)(p.y - th.ay);
+                vz[u] = (float)(p.z - th.az);
+                mi[u] = (float)p.w;
+                asm("" : "+v"(vx[u]), "+v"(vy[u]), "+v"(vz[u]), "+v"(mi[u]));
+            }
+            for (int s = 0; s < SY_WAVES; ++s) {
+#pragma unroll
+                for (int h = 0; h < SY_NB; ++h) {
+                    const int blk = ((w + s) & (SY_WAVES - 1)) * SY_NB + h;
+                    if (!((bits >> blk) & 1u)) continue;
+                    const int k = blk * 64 + lane;
+                    const double4 q = rec[k];
+                    const float wx = (float)(q.x - th.ax), wy = (float)(q.y - th.ay),
+                                wz = (float)(q.z - th.az), mj = (float)q.w;
+                    float bx = 0.f, by = 0.f, bz = 0.f;
+#pragma unroll
+                    for (int u = 0; u < MI; ++u) {
+                        const float dx = wx - vx[u], dy = wy - vy[u], dz = wz - vz[u];
+                        const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+                        const float y = __builtin_amdgcn_rsqf(r2);
+                        const float y3 = (y * y) * y;
+                        const float a = mj * y3, b = mi[u] * y3;
+                        acc[3 * u] = fmaf(a, dx, acc[3 * u]);
+                        acc[3 * u + 1] = fmaf(a, dy, acc[3 * u + 1]);
+                        acc[3 * u + 2] = fmaf(a, dz, acc[3 * u + 2]);
+                        bx = fmaf(b, dx, bx);
+                        by = fmaf(b, dy, by);
+                        bz = fmaf(b, dz, bz);
+                    }
+                    js[0][k] -= (double)bx;
+                    js[1][k] -= (double)by;
+                    js[2][k] -= (double)bz;
+                }
+                __syncthreads();
+            }
+            // Value 3 u + d; a lane ends with the sums of body u = bits 3, 2, 1
+            // of its number (partners as in lanes_sum4).
+            halve32<24, 0x140>(acc, (lane & 8) != 0);
+            halve32<12, 0x141>(acc, (lane & 4) != 0);
+            halve32<6, 0x1b>(acc, (lane & 2) != 0);
+#pragma unroll
+            for (int d = 0; d < 6; ++d) sum[d] = (double)acc[d];
+            halve64<3, 0xb1>(sum, (lane & 1) != 0);
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                sum[d] += __shfl_xor(sum[d], 16);
+                sum[d] += __shfl_xor(sum[d], 32);
+            }
+        }
+        const int u = lane & 15;
+        if (lane < 16 && i0 + u < nv) {
+            double *o = pi + 3 * (S.ioff(c) + i0 + u);
+            o[0] = sum[0];
+            o[1] = sum[1];
+            o[2] = sum[2];
+        }
+    }
+    double *o = pj + 3 * (S.joff(r) + (j0 - row0));
+#pragma unroll
+    for (int h = 0; h < SY_NB; ++h) {
+        const int k = h * SY_T + tid;
+        if (j0 + k >= row0)
+            for (int d = 0; d < 3; ++d) o[3 * (long)k + d] = js[d][k];
+    }
 }
 
 // CM_acc from the partials of k_sym_finish.
@@ -289,7 +610,54 @@ ncg_status ncg_gravity_sym(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int 
     const int cp = (c && c->present) ? 1 : 0;
     hipLaunchKernelGGL(k_sym_finish, dim3(nb), dim3(FT), 0, st, d_b, d_perm, d_nvalid, S, pi, pj, cp,
                        cp ? c->x : 0.0, cp ? c->y : 0.0, cp ? c->z : 0.0, cp ? G * c->mass : 0.0,
-                       d_central, G, d_acc, cmpart);
+                       d_central, G, (const double *)nullptr, 0, (const Scal *)nullptr, d_acc, cmpart);
+    if (d_cm_acc)
+        hipLaunchKernelGGL(k_sym_cm, dim3(1), dim3(FT), 0, st, cmpart, nb, d_cm_acc);
+    NCG_CHECK_LAUNCH();
+    return NCG_OK;
+}
+
+ncg_status ncg_gravity_mixed_sym(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int *d_perm,
+                                 const void *d_scal, const ncg_central *c, const double *d_central,
+                                 double G, double soft, double theta, double *d_acc,
+                                 double *d_cm_acc, hipStream_t st)
+{
+    const Scal *scal = static_cast<const Scal *>(d_scal);
+    // Rows a row group: few where workgroups are few (32,800 bodies, 2 / 8: 0.44
+    // and 0.50 ms), many where the partial sums weigh (262,144: 17.8 and 16.9).
+    const SymShape S = sym_shape(n, SY_NB, MI, n <= 65536 ? 2 : n <= 131072 ? 4 : 8);
+    const int ng = (int)cdiv(n, MG), nw = (int)cdiv(ng, 64);
+    double4 *jd = dbuf<double4>(ctx, "y_jd", (size_t)ng * MG);
+    double *jsig = dbuf<double>(ctx, "y_jsig", (size_t)ng * MG);
+    TileHdr *hdr = dbuf<TileHdr>(ctx, "y_hdr", ng);
+    unsigned long long *mask = dbuf<unsigned long long>(ctx, "y_mask", (size_t)ng * nw);
+    double *near = dbuf<double>(ctx, "y_near", 3 * (size_t)MNEAR * n);
+    double *pi = dbuf<double>(ctx, "y_pi", 3 * (size_t)S.islots());
+    double *pj = dbuf<double>(ctx, "y_pj", 3 * (size_t)S.jslots());
+    const int nb = (int)cdiv(n, FS);
+    double *cmpart = d_cm_acc ? dbuf<double>(ctx, "y_cm", 3 * (size_t)nb) : nullptr;
+    if (!jd || !jsig || !hdr || !mask || !near || !pi || !pj || (d_cm_acc && !cmpart))
+        return NCG_ERR_NOMEM;
+    hipLaunchKernelGGL(k_mix_records, dim3(ng), dim3(64), 0, st, d_b, d_perm, scal, G, soft, jd, jsig,
+                       hdr);
+    hipLaunchKernelGGL(k_mix_mask, dim3(ng, nw), dim3(64), 0, st, hdr, scal, nw, theta, soft, mask);
+    NCG_CHECK_LAUNCH();
+    {
+        ProfScope ps(ctx, st, "pairs_mixed");
+        if (soft != 0.0)
+            hipLaunchKernelGGL(k_mix_near<true>, dim3(ng, MNEAR), dim3(64 * NW), 0, st, jd, jsig, scal,
+                               nw, (int)n, mask, near);
+        else
+            hipLaunchKernelGGL(k_mix_near<false>, dim3(ng, MNEAR), dim3(64 * NW), 0, st, jd, jsig, scal,
+                               nw, (int)n, mask, near);
+        hipLaunchKernelGGL(k_pairs_mix, dim3((unsigned)S.workgroups()), dim3(SY_T), 0, st, jd, hdr,
+                           scal, nw, mask, S, pi, pj);
+        NCG_CHECK_LAUNCH();
+    }
+    const int cp = (c && c->present) ? 1 : 0;
+    hipLaunchKernelGGL(k_sym_finish, dim3(nb), dim3(FT), 0, st, d_b, d_perm, &scal->nvalid, S, pi, pj,
+                       cp, cp ? c->x : 0.0, cp ? c->y : 0.0, cp ? c->z : 0.0,
+                       cp ? G * c->mass : 0.0, d_central, G, near, MNEAR, scal, d_acc, cmpart);
     if (d_cm_acc)
         hipLaunchKernelGGL(k_sym_cm, dim3(1), dim3(FT), 0, st, cmpart, nb, d_cm_acc);
     NCG_CHECK_LAUNCH();

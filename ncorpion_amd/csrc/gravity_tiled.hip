@@ -5,8 +5,14 @@
 // with D^2 = |x_j - x_i|^2 + (s (R_i + R_j))^2, plus the central term
 // (physics.c:127-146), but in tile order on the vector ALUs.
 //
+// The split kernel below runs the mixed form up to NCG_STATIC_MAX_N bodies, both
+// above NCG_SYM_MAX, in the allocation-free entry point and in launch shapes of
+// the caller's; elsewhere the pairs are unordered (gravity_sym.hip, after steps
+// 1 to 3, with Hilbert keys).
+//
 // Pipeline of one evaluation (all on one stream, no host synchronisation):
-//   1. k_bbox_*      bounding box, largest radius and count of existing bodies
+//   1. k_bbox_*      bounding box, largest radius and mass, count of existing
+//                    bodies
 //   2. k_morton      mixed form: 30-bit Morton key per body over the bounding
 //                    CUBE (the same cell size on every axis, so that runs of
 //                    keys are compact in space also for a thin disk); FP64-fast
@@ -56,13 +62,7 @@
 namespace {
 
 constexpr int NT = 256;     // threads per workgroup
-
-struct Scal {           // per-evaluation scalars produced on the device
-    double bmin[3], bmax[3];
-    double rmax;
-    int nvalid;
-    int pad;
-};
+constexpr int BBP = 9;      // doubles of one partial of the bounding box
 
 // ---- 1. bounding box / count ---------------------------------------------
 __global__ __launch_bounds__(NT) void k_bbox_partial(const DBody *__restrict__ b, int n,
@@ -71,6 +71,7 @@ __global__ __launch_bounds__(NT) void k_bbox_partial(const DBody *__restrict__ b
 {
     __shared__ double sh[NT];
     double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300}, rm = 0.0, cnt = 0.0;
+    double mm = 0.0;
     for (int k = blockIdx.x * NT + threadIdx.x; k < n; k += gridDim.x * NT) {
         if (ex && !ex[k]) continue;
         const double p[3] = {b[k].x, b[k].y, b[k].z};
@@ -79,9 +80,10 @@ __global__ __launch_bounds__(NT) void k_bbox_partial(const DBody *__restrict__ b
             mx[c] = fmax(mx[c], p[c]);
         }
         rm = fmax(rm, b[k].radius);
+        mm = fmax(mm, fabs(b[k].mass));
         cnt += 1.0;
     }
-    double *o = part + 8 * blockIdx.x;
+    double *o = part + BBP * blockIdx.x;
     for (int c = 0; c < 3; ++c) {
         double v = block_reduce(mn[c], sh, 0);
         if (threadIdx.x == 0) o[c] = v;
@@ -92,6 +94,8 @@ __global__ __launch_bounds__(NT) void k_bbox_partial(const DBody *__restrict__ b
     if (threadIdx.x == 0) o[6] = v;
     v = block_reduce(cnt, sh, 2);
     if (threadIdx.x == 0) o[7] = v;
+    v = block_reduce(mm, sh, 1);
+    if (threadIdx.x == 0) o[8] = v;
 }
 
 __global__ __launch_bounds__(NT) void k_bbox_final(const double *__restrict__ part, int nparts,
@@ -99,24 +103,34 @@ __global__ __launch_bounds__(NT) void k_bbox_final(const double *__restrict__ pa
 {
     __shared__ double sh[NT];
     double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300}, rm = 0.0, cnt = 0.0;
+    double mm = 0.0;
     for (int q = threadIdx.x; q < nparts; q += NT) {
+        const double *o = part + BBP * q;
         for (int c = 0; c < 3; ++c) {
-            mn[c] = fmin(mn[c], part[8 * q + c]);
-            mx[c] = fmax(mx[c], part[8 * q + 3 + c]);
+            mn[c] = fmin(mn[c], o[c]);
+            mx[c] = fmax(mx[c], o[3 + c]);
         }
-        rm = fmax(rm, part[8 * q + 6]);
-        cnt += part[8 * q + 7];
+        rm = fmax(rm, o[6]);
+        cnt += o[7];
+        mm = fmax(mm, o[8]);
     }
+    double w = 0.0;
     for (int c = 0; c < 3; ++c) {
-        double v = block_reduce(mn[c], sh, 0);
-        if (threadIdx.x == 0) sc->bmin[c] = v;
-        v = block_reduce(mx[c], sh, 1);
-        if (threadIdx.x == 0) sc->bmax[c] = v;
+        const double lo = block_reduce(mn[c], sh, 0), hi = block_reduce(mx[c], sh, 1);
+        w = fmax(w, hi - lo);
+        if (threadIdx.x == 0) {
+            sc->bmin[c] = lo;
+            sc->bmax[c] = hi;
+        }
     }
-    double v = block_reduce(rm, sh, 1);
-    if (threadIdx.x == 0) sc->rmax = v;
-    v = block_reduce(cnt, sh, 2);
-    if (threadIdx.x == 0) sc->nvalid = (int)v;
+    const double r = block_reduce(rm, sh, 1), m = block_reduce(mm, sh, 1);
+    const double nv = block_reduce(cnt, sh, 2);
+    if (threadIdx.x == 0) {
+        sc->rmax = r;
+        sc->mmax = m;
+        sc->nvalid = (int)nv;
+        sc->lexp = exp_of(w);
+    }
 }
 
 // ---- 2. Morton keys -------------------------------------------------------
@@ -152,7 +166,8 @@ __global__ __launch_bounds__(NT) void k_morton(const DBody *__restrict__ b, int 
         v = v < 0 ? 0 : (v > 1023 ? 1023 : v);
         q[c] = (unsigned)v;
     }
-    key[k] = (expand10(q[0]) << 2) | (expand10(q[1]) << 1) | expand10(q[2]);
+    key[k] = spatial == 2 ? hilbert<10>(q[0], q[1], q[2])
+                          : (expand10(q[0]) << 2) | (expand10(q[1]) << 1) | expand10(q[2]);
 }
 
 // ---- 4. sorted records ----------------------------------------------------
@@ -687,7 +702,7 @@ static ncg_status work_order_ctx(ncg_ctx *ctx, const TiledShape &t, int32_t n, h
                                  TiledWork &w)
 {
     w.sc = dbuf<Scal>(ctx, "t_scal", 1);
-    w.bpart = dbuf<double>(ctx, "t_bpart", 8 * (size_t)t.nbb);
+    w.bpart = dbuf<double>(ctx, "t_bpart", BBP * (size_t)t.nbb);
     w.key = dbuf<unsigned>(ctx, "t_key", n);
     w.key2 = dbuf<unsigned>(ctx, "t_key2", n);
     w.idx = dbuf<int>(ctx, "t_idx", n);
@@ -719,14 +734,26 @@ static ncg_status work_eval_ctx(ncg_ctx *ctx, const TiledShape &t, int32_t n, bo
     return NCG_OK;
 }
 
-// The order of the evaluations that follow: spatial (Morton keys over the
-// bounding cube) for the mixed form, whose near/far test needs compact tiles;
+// Whether the mixed form runs by unordered pairs (gravity_sym.hip): above the
+// sizes of the allocation-free entry point, whose scratch cannot hold the
+// partial sums and whose results are this one's up to the grouping of sums; up
+// to NCG_SYM_MAX bodies (partial sums of 1.6 GB); in a launch shape of the
+// caller's the split kernel runs.  Calls of 32,800 bodies: 0.57 ms with the split
+// kernel, 0.50 by unordered pairs; of 262,144: 19.2 and 16.1.
+static bool mixed_sym_form(const ncg_ctx *ctx, int32_t n, ncg_precision prec)
+{
+    return prec == NCG_MIXED && n > NCG_STATIC_MAX_N && n <= NCG_SYM_MAX && !ctx->tiled_explicit;
+}
+
+// The order of the evaluations that follow: spatial (Morton or Hilbert keys over
+// the bounding cube) for the mixed form, whose near/far test needs compact tiles;
 // body order (existing bodies first) for the FP64-fast form.
 static ncg_status tiled_order_w(ncg_ctx *ctx, const TiledShape &t, const TiledWork &w,
                                 const DBody *d_b, int32_t n, const int32_t *d_ex,
                                 ncg_precision prec, hipStream_t st)
 {
-    const int spatial = prec == NCG_MIXED ? 1 : 0;
+    // 2: along a Hilbert curve, for the mixed form by unordered pairs.
+    const int spatial = prec == NCG_MIXED ? (mixed_sym_form(ctx, n, prec) ? 2 : 1) : 0;
     hipLaunchKernelGGL(k_bbox_partial, dim3(t.nbb), dim3(NT), 0, st, d_b, n, d_ex, w.bpart);
     hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(NT), 0, st, w.bpart, t.nbb, w.sc);
     hipLaunchKernelGGL(k_morton, dim3(cdiv(n, NT)), dim3(NT), 0, st, d_b, n, d_ex, w.sc, spatial,
@@ -868,6 +895,13 @@ ncg_status ncg_tiled_eval(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int32
         }
         return ncg_gravity_sym(ctx, d_b, n, perm, nvalid, c, d_central, G, soft, d_acc, d_cm_acc, st);
     }
+    if (mixed_sym_form(ctx, n, prec)) {
+        const int *perm = dbuf<int>(ctx, "t_perm", n);
+        const Scal *sc = dbuf<Scal>(ctx, "t_scal", 1);
+        if (!perm || !sc) return NCG_ERR_NOMEM;
+        return ncg_gravity_mixed_sym(ctx, d_b, n, perm, sc, c, d_central, G, soft,
+                                     ncg_tiled_cfg(ctx, prec, n).theta, d_acc, d_cm_acc, st);
+    }
     const TiledShape t = tiled_shape(ctx, n, prec);
     TiledWork w;
     ncg_status r = work_eval_ctx(ctx, t, n, want_cm, d_cterm, w);
@@ -960,7 +994,7 @@ static bool work_carve(unsigned char *base, size_t cap, TiledShape &t, int32_t n
     if (!w.cterm || !w.p3) return false;
     if (!tiled) return true;
     w.sc = (Scal *)take(sizeof(Scal));
-    w.bpart = (double *)take(sizeof(double) * 8 * (size_t)t.nbb);
+    w.bpart = (double *)take(sizeof(double) * BBP * (size_t)t.nbb);
     w.key = (unsigned *)take(sizeof(unsigned) * (size_t)n);
     w.key2 = (unsigned *)take(sizeof(unsigned) * (size_t)n);
     w.idx = (int *)take(sizeof(int) * (size_t)n);

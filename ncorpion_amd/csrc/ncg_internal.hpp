@@ -296,7 +296,8 @@ static inline unsigned cdiv(long a, long b) { return (unsigned)((a + b - 1) / b)
 
 // Internal launchers used across translation units.
 // Order of the tiled forms: bounding box, keys, radix sort -- Morton keys
-// for NCG_MIXED (spatially compact tiles), body order for NCG_F64_FAST.
+// for NCG_MIXED (spatially compact tiles; Hilbert keys where it runs by
+// unordered pairs), body order for NCG_F64_FAST.
 // Leaves the permutation and the count of existing bodies on the device.
 ncg_status ncg_tiled_order(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int32_t *d_ex,
                            ncg_precision prec, hipStream_t s);
@@ -323,6 +324,12 @@ constexpr int NCG_SYM_MAX = 262144;
 ncg_status ncg_gravity_sym(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int *d_perm,
                            const int *d_nvalid, const ncg_central *c, const double *d_central,
                            double G, double soft, double *d_acc, double *d_cm_acc, hipStream_t st);
+// Mixed form by unordered pairs, in the order of the last ncg_tiled_order
+// (d_perm; d_scal: its Scal record).
+ncg_status ncg_gravity_mixed_sym(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int *d_perm,
+                                 const void *d_scal, const ncg_central *c, const double *d_central,
+                                 double G, double soft, double theta, double *d_acc,
+                                 double *d_cm_acc, hipStream_t st);
 // Direct form of the fast gravity forms for 1..4096 bodies (k_small): one
 // wavefront per body; with d_cm_acc, CM_acc as a fixed-shape tree sum of the
 // terms d_cterm (3n) through d_p3 (3 * ncg_small_partials(n) doubles).

@@ -22,6 +22,22 @@ struct TileHdr {
     float smax, smin;
 };
 
+struct Scal {           // per-evaluation scalars produced on the device
+    double bmin[3], bmax[3];
+    double rmax, mmax;  // largest radius, largest |mass|
+    int nvalid;
+    int lexp;           // exponent of the box's longest edge
+};
+
+// Powers of two that the mixed form by unordered pairs scales with: positions
+// by 2^-lexp, G m by 2^-mass_exp (0 when not finite).
+__device__ inline int exp_of(double v)
+{
+    return v > 0.0 && v < 1e300 ? max(-500, min(500, ilogb(v) + 1)) : 0;
+}
+
+__device__ inline int mass_exp(const Scal &sc, double G) { return exp_of(fabs(G) * sc.mmax); }
+
 __device__ inline unsigned expand10(unsigned v)
 {
     v &= 0x3ffu;

@@ -293,3 +293,52 @@ def test_fast64_pairs_match_split_form(n, soft):
     ref = orc.vector_field_rows(b, rows, None, cen, 1.0, soft)
     ref = ref[0] if isinstance(ref, tuple) else ref
     assert rel_err(got[True, True][0][rows], ref)[0] < 1e-12
+
+
+# The mixed form by unordered pairs: from 32,769 bodies, chunks of 1024, rows of
+# 128 in groups of 64, more rows a group above 65,536 and 131,072; holes at the
+# ends; a softening above every distance of near groups; negative and far too
+# small masses.  A term's error is some six FP32 roundings (2^-24 each, half that
+# in the mean), and so is the field's in the norm, at most: 1.5e-7.
+@pytest.mark.parametrize("n,soft,odd", [(32769, 0.0, False), (33793, 0.5, True),
+                                        (65537, 0.0, True), (131073, 0.5, False)])
+def test_mixed_pairs_match_fp64(ctx, n, soft, odd):
+    import torch
+    m, R = ic.disk_c3_masses(n, n)
+    if odd:
+        m[100:230] *= -1.0
+        m[5000:5003] *= 1e-40
+    b = ic.disk(n, seed=n, masses=m, radii=R)
+    ex = (np.random.default_rng(n).uniform(size=n) > 0.07).astype(np.int32)
+    ex[[0, -1]] = 0
+    cen = (1e-3, 2e-3, -1e-3, 1.0)
+    bt, et = torch.from_numpy(b).cuda(), torch.from_numpy(ex).cuda()
+
+    def field(x, e, c, prec):
+        acc = torch.full((n, 3), 7.0, dtype=torch.float64, device="cuda")
+        cm = torch.zeros(3, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        ctx.gravity_allpairs_dev(x, acc, e, c, 1.0, soft, prec, cm)
+        ctx.synchronize()
+        return acc.cpu().numpy(), cm.cpu().numpy()
+
+    for e in (None, et):
+        on = slice(None) if e is None else ex != 0
+        a, _ = field(bt, e, None, "mixed")
+        r, _ = field(bt, e, None, "fast64")
+        if e is not None:
+            assert np.all(a[ex == 0] == 7.0)
+        assert np.linalg.norm(a[on] - r[on]) < 1.5e-7 * np.linalg.norm(r[on])
+        (a, ca), (r, cr) = field(bt, e, cen, "mixed"), field(bt, e, cen, "fast64")
+        assert np.linalg.norm(a[on] - r[on]) < 1.5e-7 * np.linalg.norm(r[on])
+        assert np.abs(ca - cr).max() < 1e-13 * np.abs(m).sum()
+    # Units that differ by powers of two: the same digits.
+    a, _ = field(bt, None, None, "mixed")
+    x = b.copy()
+    x[:, 0:3] *= 2.0 ** 90
+    x[:, 7] *= 2.0 ** 90
+    x[:, 6] *= 2.0 ** -150
+    u, _ = field(torch.from_numpy(x).cuda(), None, None, "mixed")
+    assert np.array_equal(u, a * 2.0 ** -330)
+    none, _ = field(bt, torch.zeros_like(et), None, "mixed")
+    assert np.all(none == 7.0)
