@@ -604,10 +604,30 @@ __device__ inline bool may_meet(const CollHdr &g, const CollHdr &t, double adt)
     return !(gx * gx + gy * gy + gz * gz > reach * reach);
 }
 
+// The header of a body alone (its radius rounded up).
+__device__ inline CollHdr body_hdr(const DBody &q)
+{
+    CollHdr h;
+    h.px = q.x;
+    h.py = q.y;
+    h.pz = q.z;
+    h.vx = q.vx;
+    h.vy = q.vy;
+    h.vz = q.vz;
+    h.phx = h.phy = h.phz = h.vhx = h.vhy = h.vhz = 0.f;
+    float r = (float)q.radius;
+    if ((double)r < q.radius) r = nextafterf(r, 3.0e38f);
+    h.rmax = r;
+    h.count = 1;
+    return h;
+}
+
 // One workgroup per collision unit (system, 256 slots); wavefront w takes
 // the unit's group w and tests its pairs (p, q > p in slot order) with every
-// tile from its own on that it may meet, staging each such tile in its own
-// LDS slice.  The predicate is
+// tile from its own on that it may meet, staging the tile's bodies that the
+// group may meet in its own LDS slice.  Bound by FP64 issue; a tile at a disk's
+// rim has a box that meets most groups, with few of its bodies (512 systems of
+// 256 to 8,192 bodies: 0.75 ms a pass with all of a tile's bodies, 0.35 so).  The predicate is
 // closest_approach's (collision.c:112-137; this file is compiled without FMA
 // contraction), symmetric in the pair bit for bit, with a tolerance of
 // 9.1e-13 |dt| on the contact time: candidates are a superset of the
@@ -653,19 +673,28 @@ __global__ __launch_bounds__(ENT) void k_ens_cpass(const EnsUnit *__restrict__ u
             // previous tile and before the reads below.
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
             __builtin_amdgcn_wave_barrier();
+            unsigned long long meet[TJ / WV];  // bodies that the group may meet
 #pragma unroll
             for (int r = 0; r < TJ / WV; ++r) {
                 const int l = r * WV + lane;
+                bool m = false;
                 if (l < th.count) {
                     const DBody c = jc[jb + l];
-                    tp[l] = make_double4(c.x, c.y, c.z, c.radius);
-                    tv[l] = make_double4(c.vx, c.vy, c.vz, 0.0);
-                    tk[l] = pidx[jb + l];
+                    m = jb + l > g0 && may_meet(gh, body_hdr(c), adt);
+                    if (m) {
+                        tp[l] = make_double4(c.x, c.y, c.z, c.radius);
+                        tv[l] = make_double4(c.vx, c.vy, c.vz, 0.0);
+                        tk[l] = pidx[jb + l];
+                    }
                 }
+                meet[r] = __ballot(m);
             }
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
             __builtin_amdgcn_wave_barrier();
-            for (int jj = 0; jj < th.count; ++jj) {
+#pragma unroll
+            for (int r = 0; r < TJ / WV; ++r) while (meet[r]) {
+                const int jj = r * WV + __ffsll((long long)meet[r]) - 1;
+                meet[r] &= meet[r] - 1;
                 const int q = jb + jj;
                 if (!mine || q <= p) continue;
                 const double4 cp = tp[jj], cv = tv[jj];

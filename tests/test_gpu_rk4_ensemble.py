@@ -341,6 +341,20 @@ def test_ensemble_collisions_of_clumps_crossing_within_dt(ctx):
     assert nc == total and total > 100, (nc, total)
 
 
+@pytest.mark.parametrize("backward", [False, True])
+def test_ensemble_collisions_at_tile_edges(ctx, backward):
+    """Systems at the edges of groups (64) and tiles (128), where a few large or
+    fast bodies of a tile, not the tile as a whole, reach another group."""
+    systems = []
+    for s, n in enumerate((1, 2, 63, 64, 65, 127, 128, 129, 191, 256, 257, 385)):
+        b = ic.disk(n, seed=700 + s, mass=1e-9, radius=1e-3)
+        b[::17, 7] = 0.03
+        b[5::29, 3:6] *= 1.5
+        systems.append(b)
+    nc, total = _collision_run(ctx, systems, -0.02 if backward else 0.02, 2)
+    assert nc == total and total > 10, (nc, total)
+
+
 @pytest.mark.parametrize("prec", ["fast64", "mixed"])
 def test_ensemble_with_empty_and_tiny_systems(ctx, prec):
     """Systems of 0, 1 and 2 bodies between ordinary ones (the padded slot
