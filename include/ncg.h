@@ -205,7 +205,8 @@ ncg_status ncg_gravity_allpairs_static_dev(ncg_ctx *ctx, const ncg_body *d_bodie
 /* ---------------------------------------------------------------------------
  * Brute-force collision search: replaces brute_force (collision.c:425-456).
  * The GPU tests every pair i<j of existing bodies at the given state with the
- * closest_approach predicate (collision.c:63-172) and hands the candidates to
+ * closest_approach predicate (collision.c:63-172; from 8192 bodies, those pairs
+ * that the bodies' boxes let meet within the timestep) and hands the candidates to
  * the host, which replays the reference's lexicographic (i, j) order through
  * ops: candidate pairs are confirmed with ops->test and resolved with
  * ops->resolve; after a collision every later pair that involves a modified
@@ -665,8 +666,10 @@ ncg_status ncg_cart2ell(ncg_ctx *ctx, const ncg_body *bodies, int32_t n, const i
  * per lane (1, 2, 4; 0 keeps), j-splits per i-block (0 = from the CU count,
  * -1 keeps), near/far threshold theta (<= 0 keeps), tile source (0 scalar
  * loads, 1 LDS, -1 keeps).  Results do not depend on the shape beyond FP
- * rounding of the split sums.  The autotuner (ncorpion_amd/autotune.py)
- * picks these per N.
+ * rounding of the split sums.  A shape set here selects the kernel it shapes
+ * (every ordered pair); without one, NCG_F64_FAST of 4097 to 262144 bodies and
+ * NCG_MIXED of NCG_STATIC_MAX_N + 1 to 262144 form each unordered pair once.  The
+ * autotuner (ncorpion_amd/autotune.py) picks these per N.
  */
 ncg_status ncg_set_tiling(ncg_ctx *ctx, int32_t ipl, int32_t nsplit, double theta, int32_t source);
 

@@ -1,6 +1,7 @@
 """Autotuner of the gravity launch shapes.
 
-Single systems: for each body count N (a seeded disk of that size), every
+Single systems (the split pair kernel; its theta also serves the mixed form by
+unordered pairs): for each body count N (a seeded disk of that size), every
 candidate shape -- bodies per lane, j-splits per i-block, tile source (scalar
 loads or LDS) and, for the mixed form, the near/far threshold theta -- is
 timed with HIP events around the pair kernel.  A theta is admissible only if
