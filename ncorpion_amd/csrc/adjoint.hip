@@ -286,17 +286,20 @@ __global__ __launch_bounds__(AT) void k_vjp_sym_sum(SymShape S, const double *__
 }
 
 // Central part, added to g_x / g_m; per-block partials of g_C (3) and g_M.
+// total (may be null): takes the sum's g_m instead, added to what it holds.
 __global__ __launch_bounds__(AT) void k_vjp_central(const DBody *__restrict__ b, int n,
                                                     const double *__restrict__ cen,
                                                     const double *__restrict__ lam,
                                                     const double *__restrict__ lamc, double G,
                                                     double *__restrict__ gx,
                                                     double *__restrict__ gm,
+                                                    double *__restrict__ total,
                                                     double *__restrict__ part)
 {
     __shared__ double red[4][AT];
     const int i = blockIdx.x * AT + threadIdx.x;
     double pc[4] = {0., 0., 0., 0.};
+    double gi = i < n ? gm[i] : 0.0;
     if (i < n && cen[7] != 0.0) {
         const DBody q = b[i];
         const double ex = q.x - cen[0], ey = q.y - cen[1], ez = q.z - cen[2];
@@ -315,11 +318,15 @@ __global__ __launch_bounds__(AT) void k_vjp_central(const DBody *__restrict__ b,
         gx[3 * (size_t)i + 0] += tx;
         gx[3 * (size_t)i + 1] += ty;
         gx[3 * (size_t)i + 2] += tz;
-        gm[i] += G * (cx * ex + cy * ey + cz * ez) * i3;
+        gi += G * (cx * ex + cy * ey + cz * ez) * i3;
         pc[0] = -tx;
         pc[1] = -ty;
         pc[2] = -tz;
         pc[3] = -G * (lx * ex + ly * ey + lz * ez) * i3;
+    }
+    if (i < n) {
+        if (total) total[i] += gi;
+        else gm[i] = gi;
     }
     for (int c = 0; c < 4; ++c) red[c][threadIdx.x] = pc[c];
     __syncthreads();
@@ -359,7 +366,8 @@ __global__ void k_adj_stage(int s, double h, int n, const double *__restrict__ L
                             double *__restrict__ Kv, const double *__restrict__ gX,
                             double *__restrict__ Ax, double *__restrict__ Av,
                             const double *__restrict__ cL, double *__restrict__ cK,
-                            const double *__restrict__ cg, double *__restrict__ cA)
+                            const double *__restrict__ cg, double *__restrict__ cA,
+                            double *__restrict__ gM)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const double ws[5] = {0., 1., 2., 2., 1.};
@@ -376,7 +384,8 @@ __global__ void k_adj_stage(int s, double h, int n, const double *__restrict__ L
             }
         }
     } else if (i == n && cK) {
-        // central: cL = ybar' (6), cK = Kbar (6), cg = g_C (3), cA = ybar (6)
+        // central: cL = ybar' (6), cK = Kbar (6), cg = g_C (3) and g_M, cA = ybar (6)
+        *gM += cg[3];
         for (int d = 0; d < 3; ++d) {
             const double g = cg[d], kx = cK[d];
             cA[d] += g;
@@ -451,12 +460,6 @@ __global__ void k_adj_zero(double *__restrict__ a, int n)
     if (i < n) a[i] = 0.0;
 }
 
-__global__ void k_add(double *__restrict__ a, const double *__restrict__ b, int n)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) a[i] += b[i];
-}
-
 }  // namespace
 
 // Bodies for which the pair part runs by unordered pairs: 114 us against 112 by
@@ -506,9 +509,8 @@ static ncg_status vjp_impl(ncg_ctx *ctx, const DBody *b, int32_t n, const double
         hipLaunchKernelGGL(k_vjp_reduce, dim3(nb), dim3(AT), 0, st, pp, nsplit, (int)n, G, gx, gm_tmp);
     }
     hipLaunchKernelGGL(k_vjp_central, dim3(nb), dim3(AT), 0, st, b, (int)n, cen, lam, lamc, G, gx,
-                       gm_tmp, part);
+                       gm_tmp, accumulate ? gm : nullptr, part);
     hipLaunchKernelGGL(k_sum4, dim3(1), dim3(AT), 0, st, part, nb, gcm, 0);
-    if (accumulate) hipLaunchKernelGGL(k_add, dim3(cdiv(n, 256)), dim3(256), 0, st, gm, gm_tmp, (int)n);
     NCG_CHECK_LAUNCH();
     return NCG_OK;
 }
@@ -546,15 +548,19 @@ static ncg_status fwd_step_store(ncg_ctx *ctx, DBody *y, int32_t n, double *c0, 
     ncg_central cf = {};
     cf.present = 1;  // the device central record's own flag decides (k_finish reads it)
     for (int s = 0; s < 4; ++s) {
-        const DBody *src = s == 0 ? y : Y;
-        const double *dc = s == 0 ? c0 : Yc;
-        if (Ys) {
-            NCG_HIP(hipMemcpyAsync(Ys + (size_t)s * n, src, sizeof(DBody) * n, hipMemcpyDeviceToDevice, st));
-            NCG_HIP(hipMemcpyAsync(Ycs + 8 * s, dc, sizeof(double) * 8, hipMemcpyDeviceToDevice, st));
+        // Stage states: stored ones in their places (stage s writes s + 1's).
+        DBody *at = Ys ? Ys + (size_t)s * n : Y, *next = Ys && s < 3 ? at + n : at;
+        double *atc = Ycs ? Ycs + 8 * s : Yc, *nextc = Ycs && s < 3 ? atc + 8 : atc;
+        if (Ys && s == 0) {
+            NCG_HIP(hipMemcpyAsync(Ys, y, sizeof(DBody) * n, hipMemcpyDeviceToDevice, st));
+            NCG_HIP(hipMemcpyAsync(Ycs, c0, sizeof(double) * 8, hipMemcpyDeviceToDevice, st));
         }
+        const DBody *src = s == 0 ? y : at;
+        const double *dc = s == 0 ? c0 : atc;
         r = ncg_tiled_eval(ctx, src, n, nullptr, &cf, dc, G, soft, NCG_F64_FAST, acc, nullptr, cm, st);
         if (r != NCG_OK) return r;
-        r = ncg_rk4_stage_launch(ctx, s, dt, n, nullptr, y, Y, acc, sx, sv, c0, Yc, cm, sc, st);
+        r = ncg_rk4_stage_launch(ctx, s, dt, n, nullptr, y, at, next, acc, sx, sv, c0, atc, nextc, cm, sc,
+                                 st);
         if (r != NCG_OK) return r;
     }
     return NCG_OK;
@@ -578,10 +584,10 @@ static ncg_status adjoint_backward(ncg_ctx *ctx, const DBody *ck, const double *
     double *Ax = dbuf<double>(ctx, "a_Ax", 3 * (size_t)n), *Av = dbuf<double>(ctx, "a_Av", 3 * (size_t)n);
     double *Kx = dbuf<double>(ctx, "a_Kx", 3 * (size_t)n), *Kv = dbuf<double>(ctx, "a_Kv", 3 * (size_t)n);
     double *gX = dbuf<double>(ctx, "a_gX", 3 * (size_t)n);
-    double *cst = dbuf<double>(ctx, "a_cst", 32);  // cL[6] cK[6] cA[6] gcm[4] lamc[3]
+    double *cst = dbuf<double>(ctx, "a_cst", 32);  // cL[6] cK[6] cA[6] gcm[4] gC[4]
     if (!y || !c || !Ys || !Ycs || !Lx || !Lv || !Ax || !Av || !Kx || !Kv || !gX || !cst)
         return NCG_ERR_NOMEM;
-    double *cL = cst, *cK = cst + 6, *cA = cst + 12, *gcm = cst + 18, *lamc = cst + 22;
+    double *cL = cst, *cK = cst + 6, *cA = cst + 12, *gcm = cst + 18, *gC = cst + 22;
     // Final cotangent: d_gfinal is (x, v) per body, 6n, interleaved x,y,z,vx,vy,vz.
     hipLaunchKernelGGL(k_adj_split, dim3(cdiv(n + 1, 256)), dim3(256), 0, st, d_gfinal,
                        d_gcentral_final, (int)n, Lx, Lv, cL);
@@ -604,19 +610,17 @@ static ncg_status adjoint_backward(ncg_ctx *ctx, const DBody *ck, const double *
                                Lv, Kx, Kv, Ax, Av, cL, cK, cA);
             for (int s = 4; s >= 1; --s) {
                 // VJP at stage s with cotangent Kbar_s.v (bodies) and Kbar_s.v (central).
-                NCG_HIP(hipMemcpyAsync(lamc, cK + 3, sizeof(double) * 3, hipMemcpyDeviceToDevice, st));
-                double *gC = cst + 26;  // g_C (3) + g_M (1) of this stage
                 ncg_status r = vjp_impl(ctx, Yst + (size_t)(s - 1) * n, n, Yct + 8 * (s - 1), G, soft,
-                                        Kv, lamc, gX, d_gm, gC, true, st);
+                                        Kv, cK + 3, gX, d_gm, gC, true, st);
                 if (r != NCG_OK) return r;
                 hipLaunchKernelGGL(k_adj_stage, dim3(cdiv(n + 1, 256)), dim3(256), 0, st, s, h, (int)n,
-                                   Lx, Lv, Kx, Kv, gX, Ax, Av, cL, cK, gC, cA);
-                hipLaunchKernelGGL(k_add, dim3(1), dim3(64), 0, st, gcm + 3, gC + 3, 1);
+                                   Lx, Lv, Kx, Kv, gX, Ax, Av, cL, cK, gC, cA, gcm + 3);
                 NCG_CHECK_LAUNCH();
             }
-            NCG_HIP(hipMemcpyAsync(Lx, Ax, sizeof(double) * 3 * n, hipMemcpyDeviceToDevice, st));
-            NCG_HIP(hipMemcpyAsync(Lv, Av, sizeof(double) * 3 * n, hipMemcpyDeviceToDevice, st));
-            NCG_HIP(hipMemcpyAsync(cL, cA, sizeof(double) * 6, hipMemcpyDeviceToDevice, st));
+            // The state adjoint is the next step's cotangent.
+            std::swap(Lx, Ax);
+            std::swap(Lv, Av);
+            std::swap(cL, cA);
         }
     }
     // Outputs: g0 interleaved (x, v) per body; central (x, v) and g_M.

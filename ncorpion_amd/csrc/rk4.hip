@@ -48,16 +48,17 @@ namespace {
 
 constexpr int NT = 256;
 
-// Stage s of RK4 (s = 0..3).  Y holds the stage state used by evaluation s;
-// acc its acceleration.  After the update Y holds the state for stage s+1, or
-// (s == 3) y0 holds the new state.
+// Stage s of RK4 (s = 0..3).  Y holds the stage state used by evaluation s
+// (s == 0: y0 does); acc its acceleration.  After the update Yn, which may be Y,
+// holds the state for stage s+1, or (s == 3) y0 holds the new state; Yc and Ycn
+// likewise for the central body.
 __global__ __launch_bounds__(NT) void k_rk4_stage(int s, double dt, int n,
                                                   const int32_t *__restrict__ ex,
-                                                  DBody *__restrict__ y0, DBody *__restrict__ Y,
+                                                  DBody *__restrict__ y0, const DBody *Y, DBody *Yn,
                                                   const double *__restrict__ acc,
                                                   double *__restrict__ sx, double *__restrict__ sv,
-                                                  double *__restrict__ c0, double *__restrict__ Yc,
-                                                  const double *__restrict__ cm_acc,
+                                                  double *__restrict__ c0, const double *Yc,
+                                                  double *Ycn, const double *__restrict__ cm_acc,
                                                   double *__restrict__ sc)
 {
     const int i = blockIdx.x * NT + threadIdx.x;
@@ -85,7 +86,7 @@ __global__ __launch_bounds__(NT) void k_rk4_stage(int s, double dt, int n,
             ny.vx = b0.vx + h * a[0];
             ny.vy = b0.vy + h * a[1];
             ny.vz = b0.vz + h * a[2];
-            Y[i] = ny;
+            Yn[i] = ny;
         } else {
             DBody nb = b0;
             const double f = dt / 6.0;
@@ -98,6 +99,7 @@ __global__ __launch_bounds__(NT) void k_rk4_stage(int s, double dt, int n,
             y0[i] = nb;
         }
     }
+    if (i == 0 && c0[7] == 0.0 && s < 3) Ycn[7] = 0.0;
     if (i == 0 && c0[7] != 0.0) {
         const double *cs = s == 0 ? c0 : Yc;
         double kx[3], kv[3];
@@ -109,11 +111,12 @@ __global__ __launch_bounds__(NT) void k_rk4_stage(int s, double dt, int n,
             for (int d = 0; d < 3; ++d) {
                 sc[d] = kx[d];
                 sc[3 + d] = kv[d];
-                Yc[d] = c0[d] + h * cs[3 + d];
-                Yc[3 + d] = c0[3 + d] + h * cm_acc[d];
+                const double v = cs[3 + d];
+                Ycn[d] = c0[d] + h * v;
+                Ycn[3 + d] = c0[3 + d] + h * cm_acc[d];
             }
-            Yc[6] = c0[6];
-            Yc[7] = c0[7];
+            Ycn[6] = c0[6];
+            Ycn[7] = c0[7];
         } else {
             const double f = dt / 6.0;
             for (int d = 0; d < 3; ++d) {
@@ -127,12 +130,12 @@ __global__ __launch_bounds__(NT) void k_rk4_stage(int s, double dt, int n,
 }  // namespace
 
 ncg_status ncg_rk4_stage_launch(ncg_ctx *ctx, int s, double dt, int32_t n, const int32_t *ex,
-                                DBody *y0, DBody *Y, const double *acc, double *sx, double *sv,
-                                double *c0, double *Yc, const double *cm, double *sc,
-                                hipStream_t st)
+                                DBody *y0, const DBody *Y, DBody *Yn, const double *acc, double *sx,
+                                double *sv, double *c0, const double *Yc, double *Ycn,
+                                const double *cm, double *sc, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_rk4_stage, dim3(cdiv(n, NT)), dim3(NT), 0, st, s, dt, (int)n, ex, y0, Y, acc,
-                       sx, sv, c0, Yc, cm, sc);
+    hipLaunchKernelGGL(k_rk4_stage, dim3(cdiv(n, NT)), dim3(NT), 0, st, s, dt, (int)n, ex, y0, Y, Yn,
+                       acc, sx, sv, c0, Yc, Ycn, cm, sc);
     NCG_CHECK_LAUNCH();
     return NCG_OK;
 }
@@ -160,7 +163,7 @@ static ncg_status rk4_body(ncg_ctx *ctx, DBody *y0, int32_t n, const int32_t *ex
                                       central_present ? cm : nullptr, st);
         if (r != NCG_OK) return r;
         hipLaunchKernelGGL(k_rk4_stage, dim3(cdiv(n, NT)), dim3(NT), 0, st, s, dt, (int)n, ex, y0, Y,
-                           acc, sx, sv, c0, Yc, cm, sc);
+                           Y, acc, sx, sv, c0, Yc, Yc, cm, sc);
         NCG_CHECK_LAUNCH();
     }
     return NCG_OK;

@@ -110,6 +110,31 @@ def test_rk4_adjoint_matches_torch_autograd(ctx, nsteps, K):
         assert float((w - u).abs().max()) <= 1e-9 * scale, (u, w)
 
 
+@pytest.mark.parametrize("n", [96, 10241])
+def test_rk4_adjoint_without_central_body_after_one_with(ctx, n):
+    """The recomputed stages write their states and central records in place: a
+    run without a central body is not touched by an earlier one's, and its
+    gradients are those of a central body without mass."""
+    torch = tt()
+    G, soft, h, nsteps = 1.0, 0.01, 2 * math.pi / 256, 3
+    b = disk(n, 5)
+    rng = np.random.default_rng(6)
+    wx, wv = (torch.tensor(rng.normal(size=(n, 3)), device="cuda") for _ in range(2))
+    got = []
+    for mass, present in ((1.0, 1.0), (0.0, 0.0), (0.0, 1.0)):
+        from ncorpion_amd.autograd import RK4Trajectory
+        x, v, m = (torch.tensor(b[:, k], requires_grad=True, device="cuda")
+                   for k in (slice(0, 3), slice(3, 6), 6))
+        R = torch.tensor(b[:, 7], device="cuda")
+        cen = torch.tensor([0, 0, 0, 0, 0, 0, mass, present], dtype=torch.float64, device="cuda")
+        xT, vT, _ = RK4Trajectory.apply(x, v, m, R, cen, G, soft, h, nsteps, 2, ctx)
+        got.append(torch.autograd.grad((xT * wx).sum() + (vT * wv).sum(), (x, v, m)))
+    for u, w in zip(got[2], got[1]):
+        scale = float(u.abs().max())
+        assert float((w - u).abs().max()) <= 1e-12 * scale
+    assert float((got[0][0] - got[1][0]).abs().max()) > 0.0
+
+
 def _fd_setup(ctx, n, nsteps, K, mass, radius, seed, soft):
     """Loss = mean squared distance of final positions to a seeded target
     (sigma 1e-3).  Returns (loss(bodies), adjoint gradients g0, gm, initial
