@@ -63,10 +63,13 @@ __device__ inline void window_quotients(double *n, double r2)
     y = __builtin_fma(y, __builtin_fma(-D3, y, 1.0), y);
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
+        // With r = n - D3 q, the quotient is r y + q and its negative -(r y + q),
+        // the same rounding.  A zero n leaves r = 0, whose sign decides that of
+        // the result: from fma(-D3, q, n) it is +0, which keeps the sign in -r y
+        // - q, and from fma(D3, q, -n), there -r, it keeps the sign in r y + q.
         const double q = n[c] * y;
-        const double r = __builtin_fma(-D3, q, n[c]);
-        // NEG: -(r y + q) is the same rounding, the sign of a zero turned too.
-        n[c] = NEG ? __builtin_fma(-r, y, -q) : __builtin_fma(r, y, q);
+        if (NEG) n[c] = __builtin_fma(-__builtin_fma(-D3, q, n[c]), y, -q);
+        else n[c] = __builtin_fma(-__builtin_fma(D3, q, -n[c]), y, q);
     }
 }
 

@@ -252,6 +252,28 @@ def test_exact_bitwise_edges(ctx, n, kind, soft):
         assert np.array_equal(bits(cm), bits(rcm))
 
 
+# A flat disk with both zeros on the axis and the central body in its plane: the
+# z sum of the last body at +0 is -0 (its central term, or start value, and
+# every term after it), which a term of +0 for one of -0 would turn.
+@pytest.mark.parametrize("n", [5, 193, 577, 1153])
+def test_exact_keeps_the_sign_of_zero(ctx, n):
+    b = _exact_edge_bodies(n, "flat")
+    b[:, 2] = 0.0
+    b[n // 4:, 2] = -0.0
+    ex = (np.random.default_rng(n).uniform(size=n) > 0.1).astype(np.int32)
+    ex[n // 4 - 1] = 1
+    cen = (0.1, 0.2, 0.0, 1.0)
+    for e in (None, ex):
+        on = np.ones(n, bool) if e is None else e != 0
+        ref, rcm = orc.vector_field_brute(b, e, cen, 1.0, 0.0)
+        assert np.signbit(ref[n // 4 - 1, 2]) and np.all(ref[on, 2] == 0.0)
+        acc, cm = ctx.gravity_allpairs(b, e, cen, 1.0, 0.0, "exact")
+        assert np.array_equal(bits(acc[on]), bits(ref[on]))
+        assert np.array_equal(bits(cm), bits(rcm))
+        got = ctx.gravity_allpairs_from(b, central_start(b, on, cen, 1.0), e, 1.0, 0.0, "exact")
+        assert np.array_equal(bits(got[on]), bits(ref[on]))
+
+
 # The FP64-fast form by unordered pairs: chunks of 1024 bodies, row groups of 64
 # to 512 (more rows a group above 20,000 and 65,536 bodies), remainders of every
 # kind, holes at the ends; both softening kernels; the split kernel in a shape of
