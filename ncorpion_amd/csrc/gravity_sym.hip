@@ -162,6 +162,7 @@ __global__ __launch_bounds__(FT) void k_sym_finish(const DBody *__restrict__ b,
                                                    double cy, double cz, double mu,
                                                    const double *__restrict__ dcen, double G,
                                                    const double *__restrict__ near, int nnear,
+                                                   const int *__restrict__ far,
                                                    const Scal *__restrict__ scal,
                                                    double *__restrict__ acc,
                                                    double *__restrict__ cmpart)
@@ -169,15 +170,20 @@ __global__ __launch_bounds__(FT) void k_sym_finish(const DBody *__restrict__ b,
     __shared__ double sh[FQ][3 * FS];
     const int nv = nvalid ? *nvalid : S.n;
     const int s0 = blockIdx.x * FS, tid = threadIdx.x;
+    const bool pairs = !far || *far;  // the pair kernel wrote sums
     for (int item = tid; item < FQ * 3 * FS; item += FT) {
         const int q = item / (3 * FS), e = item % (3 * FS);
         const int s = s0 + e / 3;
         double a = 0.0;
         if (s < nv) {
             const int c1 = (nv + SY_C - 1) / SY_C, r1 = s / S.W + 1;
-            a = share_sum<FQ>(s / SY_C + q, c1, [&](int c) { return pi[3 * (S.ioff(c) + s0) + e]; });
-            a += share_sum<FQ>(q, r1,
-                           [&](int r) { return pj[3 * (S.joff(r) + s0 - (long)r * S.W) + e]; });
+            if (pairs) {
+                a = share_sum<FQ>(s / SY_C + q, c1,
+                                  [&](int c) { return pi[3 * (S.ioff(c) + s0) + e]; });
+                a += share_sum<FQ>(q, r1, [&](int r) {
+                    return pj[3 * (S.joff(r) + s0 - (long)r * S.W) + e];
+                });
+            }
             // The mixed form's near terms.
             if (q < nnear) a += near[3 * ((size_t)q * S.n + s0) + e];
         }
@@ -265,8 +271,9 @@ __global__ __launch_bounds__(FT) void k_sym_records(const DBody *__restrict__ b,
 // twice as often); sums over all lanes in FP32: error +10 %.
 constexpr int MI = 16;            // bodies i of a wavefront
 constexpr int MG = 64;            // bodies of a group: half a row of wavefronts
-constexpr int MNEAR = 4;          // partial sums of a body's near terms
-constexpr int NW = 8;             // wavefronts that form one
+constexpr int MNEAR = 16;         // partial sums of a body's near terms
+constexpr int NW = 4;             // wavefronts that form one
+static_assert(MNEAR <= FQ && MNEAR * NW == 64, "one share of k_sym_finish, one bit of a word each");
 constexpr int MROW = SY_WAVES * MI;
 static_assert(MROW == 2 * MG, "a row of wavefronts is two groups");
 
@@ -275,10 +282,11 @@ __global__ __launch_bounds__(64) void k_mix_records(const DBody *__restrict__ b,
                                                     const Scal *__restrict__ scal, double G,
                                                     double soft, double4 *__restrict__ jd,
                                                     double *__restrict__ jsig,
-                                                    TileHdr *__restrict__ hdr)
+                                                    TileHdr *__restrict__ hdr, int *__restrict__ far)
 {
     const Scal S = *scal;
     const int g = blockIdx.x, lane = threadIdx.x, s = g * MG + lane;
+    if (g == 0 && lane == 0) *far = 0;
     if (g * MG >= S.nvalid) return;
     const DBody q = b[perm[min(s, S.nvalid - 1)]];
     const double gm = G * q.mass;
@@ -338,10 +346,11 @@ __device__ inline bool near_pair(const TileHdr &a, const TileHdr &b, double thet
     return !far;
 }
 
-// Bit h of group g's row: g and h are far.
+// Bit h of group g's row: g and h are far; *any: some two groups are.
 __global__ __launch_bounds__(64) void k_mix_mask(const TileHdr *__restrict__ hdr,
                                                  const Scal *__restrict__ scal, int nw, double theta,
-                                                 double soft, unsigned long long *__restrict__ mask)
+                                                 double soft, unsigned long long *__restrict__ mask,
+                                                 int *__restrict__ any)
 {
     const int ng = (scal->nvalid + MG - 1) / MG;
     const int g = blockIdx.x, h = blockIdx.y * 64 + (int)threadIdx.x;
@@ -353,21 +362,19 @@ __global__ __launch_bounds__(64) void k_mix_mask(const TileHdr *__restrict__ hdr
         far = !near_pair(a, b, theta, eps * eps * 67108864.0 /* 2^26 */);
     }
     const unsigned long long bits = __ballot(far);
-    if (threadIdx.x == 0) mask[(size_t)g * nw + blockIdx.y] = bits;
+    if (threadIdx.x == 0) {
+        mask[(size_t)g * nw + blockIdx.y] = bits;
+        if (bits) *any = 1;
+    }
 }
 
-// Near terms: body i per lane, the near groups h = share modulo MNEAR NW with
-// wave-uniform addresses.  FP64 issue; 32 shares, because a few groups (the
-// sparse rim of a disk) are near to most others and last: with 8 shares the
-// kernel took 2.32 ms at 262,144 bodies and 0.98 at 65,536, with 32 1.29 and 0.28.
-constexpr unsigned long long near_step(int shares)
-{
-    unsigned long long v = 0;
-    for (int k = 0; k < 64; k += shares) v |= 1ull << k;
-    return v;
-}
-constexpr unsigned long long NEAR_STEP = near_step(MNEAR * NW);
-
+// Near terms: body i per lane, the near groups h = share modulo 64 with
+// wave-uniform addresses.  FP64 issue.  So many shares because a few groups (the
+// sparse rim of a disk) are near to most others and last (8 shares: 2.32 ms at
+// 262,144 bodies and 0.98 at 65,536, 32: 1.29 and 0.28), and because fewer leave
+// compute units idle at the end where all groups are near to all (softening
+// lengths above some 1e-4 of the system; 45,983 bodies: 1.64 ms with 32 shares in
+// workgroups of 8 wavefronts, 1.58 so).
 template <bool SOFT>
 __global__ __launch_bounds__(64 * NW) void k_mix_near(const double4 *__restrict__ jd,
                                                  const double *__restrict__ jsig,
@@ -385,27 +392,22 @@ __global__ __launch_bounds__(64 * NW) void k_mix_near(const double4 *__restrict_
     const double si = SOFT ? jsig[i] : 0.0;
     double ax = 0.0, ay = 0.0, az = 0.0;
     const unsigned long long *row = mask + (size_t)g * nw;
-    for (int w = 0; w * 64 < ng; ++w) {
-        unsigned long long bits = ~row[w] & (NEAR_STEP << share);
-        if (w * 64 + 64 > ng) bits &= ~0ull >> (w * 64 + 64 - ng);
-        while (bits) {
-            const int h = w * 64 + __ffsll((long long)bits) - 1;
-            bits &= bits - 1;
-            const int jb = h * MG, cnt = min(MG, nv - jb);
-            if (h == g) {
-                for (int jj = 0; jj < cnt; ++jj)
-                    near_term_self<1, SOFT>(jd[jb + jj], SOFT ? jsig[jb + jj] : 0.0, jb + jj, i, MG,
-                                            &me.x, &me.y, &me.z, &si, &ax, &ay, &az);
-            } else if (cnt == MG) {
+    for (int h = share; h < ng; h += 64) {
+        if ((row[h >> 6] >> share) & 1) continue;
+        const int jb = h * MG, cnt = min(MG, nv - jb);
+        if (h == g) {
+            for (int jj = 0; jj < cnt; ++jj)
+                near_term_self<1, SOFT>(jd[jb + jj], SOFT ? jsig[jb + jj] : 0.0, jb + jj, i, MG, &me.x,
+                                        &me.y, &me.z, &si, &ax, &ay, &az);
+        } else if (cnt == MG) {
 #pragma unroll 4
-                for (int jj = 0; jj < MG; ++jj)
-                    near_term<1, SOFT>(jd[jb + jj], SOFT ? jsig[jb + jj] : 0.0, &me.x, &me.y, &me.z,
-                                       &si, &ax, &ay, &az);
-            } else {
-                for (int jj = 0; jj < cnt; ++jj)
-                    near_term<1, SOFT>(jd[jb + jj], SOFT ? jsig[jb + jj] : 0.0, &me.x, &me.y, &me.z,
-                                       &si, &ax, &ay, &az);
-            }
+            for (int jj = 0; jj < MG; ++jj)
+                near_term<1, SOFT>(jd[jb + jj], SOFT ? jsig[jb + jj] : 0.0, &me.x, &me.y, &me.z, &si,
+                                   &ax, &ay, &az);
+        } else {
+            for (int jj = 0; jj < cnt; ++jj)
+                near_term<1, SOFT>(jd[jb + jj], SOFT ? jsig[jb + jj] : 0.0, &me.x, &me.y, &me.z, &si,
+                                   &ax, &ay, &az);
         }
     }
     sum[wv][0][lane] = ax;
@@ -441,11 +443,13 @@ __global__ __launch_bounds__(SY_T, 4) void k_pairs_mix(const double4 *__restrict
                                                        const TileHdr *__restrict__ hdr,
                                                        const Scal *__restrict__ scal, int nw,
                                                        const unsigned long long *__restrict__ mask,
-                                                       SymShape S, double *__restrict__ pi,
+                                                       const int *__restrict__ far, SymShape S,
+                                                       double *__restrict__ pi,
                                                        double *__restrict__ pj)
 {
     __shared__ double4 rec[SY_C];
     __shared__ double js[3][SY_C];
+    if (!*far) return;  // no two groups are far: nothing to form or to add
     int r, c;
     sym_place(S, blockIdx.x, r, c);
     const int nv = scal->nvalid, tid = threadIdx.x, lane = tid & 63;
@@ -610,7 +614,8 @@ ncg_status ncg_gravity_sym(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int 
     const int cp = (c && c->present) ? 1 : 0;
     hipLaunchKernelGGL(k_sym_finish, dim3(nb), dim3(FT), 0, st, d_b, d_perm, d_nvalid, S, pi, pj, cp,
                        cp ? c->x : 0.0, cp ? c->y : 0.0, cp ? c->z : 0.0, cp ? G * c->mass : 0.0,
-                       d_central, G, (const double *)nullptr, 0, (const Scal *)nullptr, d_acc, cmpart);
+                       d_central, G, (const double *)nullptr, 0, (const int *)nullptr,
+                       (const Scal *)nullptr, d_acc, cmpart);
     if (d_cm_acc)
         hipLaunchKernelGGL(k_sym_cm, dim3(1), dim3(FT), 0, st, cmpart, nb, d_cm_acc);
     NCG_CHECK_LAUNCH();
@@ -632,15 +637,17 @@ ncg_status ncg_gravity_mixed_sym(ncg_ctx *ctx, const DBody *d_b, int32_t n, cons
     TileHdr *hdr = dbuf<TileHdr>(ctx, "y_hdr", ng);
     unsigned long long *mask = dbuf<unsigned long long>(ctx, "y_mask", (size_t)ng * nw);
     double *near = dbuf<double>(ctx, "y_near", 3 * (size_t)MNEAR * n);
+    int *far = dbuf<int>(ctx, "y_far", 1);
     double *pi = dbuf<double>(ctx, "y_pi", 3 * (size_t)S.islots());
     double *pj = dbuf<double>(ctx, "y_pj", 3 * (size_t)S.jslots());
     const int nb = (int)cdiv(n, FS);
     double *cmpart = d_cm_acc ? dbuf<double>(ctx, "y_cm", 3 * (size_t)nb) : nullptr;
-    if (!jd || !jsig || !hdr || !mask || !near || !pi || !pj || (d_cm_acc && !cmpart))
+    if (!jd || !jsig || !hdr || !mask || !near || !far || !pi || !pj || (d_cm_acc && !cmpart))
         return NCG_ERR_NOMEM;
     hipLaunchKernelGGL(k_mix_records, dim3(ng), dim3(64), 0, st, d_b, d_perm, scal, G, soft, jd, jsig,
-                       hdr);
-    hipLaunchKernelGGL(k_mix_mask, dim3(ng, nw), dim3(64), 0, st, hdr, scal, nw, theta, soft, mask);
+                       hdr, far);
+    hipLaunchKernelGGL(k_mix_mask, dim3(ng, nw), dim3(64), 0, st, hdr, scal, nw, theta, soft, mask,
+                       far);
     NCG_CHECK_LAUNCH();
     {
         ProfScope ps(ctx, st, "pairs_mixed");
@@ -651,13 +658,13 @@ ncg_status ncg_gravity_mixed_sym(ncg_ctx *ctx, const DBody *d_b, int32_t n, cons
             hipLaunchKernelGGL(k_mix_near<false>, dim3(ng, MNEAR), dim3(64 * NW), 0, st, jd, jsig, scal,
                                nw, (int)n, mask, near);
         hipLaunchKernelGGL(k_pairs_mix, dim3((unsigned)S.workgroups()), dim3(SY_T), 0, st, jd, hdr,
-                           scal, nw, mask, S, pi, pj);
+                           scal, nw, mask, far, S, pi, pj);
         NCG_CHECK_LAUNCH();
     }
     const int cp = (c && c->present) ? 1 : 0;
     hipLaunchKernelGGL(k_sym_finish, dim3(nb), dim3(FT), 0, st, d_b, d_perm, &scal->nvalid, S, pi, pj,
                        cp, cp ? c->x : 0.0, cp ? c->y : 0.0, cp ? c->z : 0.0,
-                       cp ? G * c->mass : 0.0, d_central, G, near, MNEAR, scal, d_acc, cmpart);
+                       cp ? G * c->mass : 0.0, d_central, G, near, MNEAR, far, scal, d_acc, cmpart);
     if (d_cm_acc)
         hipLaunchKernelGGL(k_sym_cm, dim3(1), dim3(FT), 0, st, cmpart, nb, d_cm_acc);
     NCG_CHECK_LAUNCH();

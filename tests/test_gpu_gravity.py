@@ -364,3 +364,25 @@ def test_mixed_pairs_match_fp64(ctx, n, soft, odd):
     assert np.array_equal(u, a * 2.0 ** -330)
     none, _ = field(bt, torch.zeros_like(et), None, "mixed")
     assert np.all(none == 7.0)
+
+
+# Softening beyond the system: every pair of groups is near, the far kernel forms
+# nothing and its sums (an earlier call's) are left out.  FP64 sums of 3e4 terms:
+# ~sqrt(n) ulps, 1e-13.
+@pytest.mark.parametrize("n", [32769, 40001])
+def test_mixed_pairs_all_near(ctx, n):
+    import torch
+    m, R = ic.disk_c3_masses(n, n)
+    bt = torch.from_numpy(ic.disk(n, seed=n, masses=m, radii=R)).cuda()
+
+    def field(soft, prec):
+        acc = torch.zeros((n, 3), dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        ctx.gravity_allpairs_dev(bt, acc, None, None, 1.0, soft, prec)
+        ctx.synchronize()
+        return acc.cpu().numpy()
+
+    far = field(0.0, "mixed")
+    near, ref = field(10.0, "mixed"), field(10.0, "fast64")
+    assert np.linalg.norm(near - ref) < 1e-13 * np.linalg.norm(ref)
+    assert np.array_equal(field(0.0, "mixed"), far)
