@@ -49,16 +49,22 @@ namespace {
 constexpr int NT = 256;
 
 // Stage s of RK4 (s = 0..3).  Y holds the stage state used by evaluation s
-// (s == 0: y0 does); acc its acceleration.  After the update Yn, which may be Y,
-// holds the state for stage s+1, or (s == 3) y0 holds the new state; Yc and Ycn
-// likewise for the central body.
+// (s == 0: y0 does); acc its acceleration.  After the update Yn, or Y (INPLACE:
+// Yn is not read), holds the state for stage s+1, or (s == 3) y0 holds the new
+// state; Yc and Ycn likewise for the central body.  Every pointer is its own
+// array, and body 0's lane loads the central body's operands before it stores
+// anything: with one kernel for both updates, whose Y and Yn may be one, each load
+// waited for the stores before it (2000 bodies: 3.70 us a stage against 3.37).
+template <bool INPLACE>
 __global__ __launch_bounds__(NT) void k_rk4_stage(int s, double dt, int n,
                                                   const int32_t *__restrict__ ex,
-                                                  DBody *__restrict__ y0, const DBody *Y, DBody *Yn,
+                                                  DBody *__restrict__ y0, DBody *__restrict__ Y,
+                                                  DBody *__restrict__ Yn,
                                                   const double *__restrict__ acc,
                                                   double *__restrict__ sx, double *__restrict__ sv,
-                                                  double *__restrict__ c0, const double *Yc,
-                                                  double *Ycn, const double *__restrict__ cm_acc,
+                                                  double *__restrict__ c0, double *__restrict__ Yc,
+                                                  double *__restrict__ Ycn,
+                                                  const double *__restrict__ cm_acc,
                                                   double *__restrict__ sc)
 {
     const int i = blockIdx.x * NT + threadIdx.x;
@@ -86,7 +92,7 @@ __global__ __launch_bounds__(NT) void k_rk4_stage(int s, double dt, int n,
             ny.vx = b0.vx + h * a[0];
             ny.vy = b0.vy + h * a[1];
             ny.vz = b0.vz + h * a[2];
-            Yn[i] = ny;
+            (INPLACE ? Y : Yn)[i] = ny;
         } else {
             DBody nb = b0;
             const double f = dt / 6.0;
@@ -99,30 +105,40 @@ __global__ __launch_bounds__(NT) void k_rk4_stage(int s, double dt, int n,
             y0[i] = nb;
         }
     }
-    if (i == 0 && c0[7] == 0.0 && s < 3) Ycn[7] = 0.0;
-    if (i == 0 && c0[7] != 0.0) {
-        const double *cs = s == 0 ? c0 : Yc;
-        double kx[3], kv[3];
+    if (i != 0) return;
+    double *const out = INPLACE ? Yc : Ycn;
+    if (c0[7] == 0.0) {
+        if (s < 3) out[7] = 0.0;  // an earlier run's record would count as present
+        return;
+    }
+    // Sums of an earlier stage (s == 0: not used).
+    double c[7], v[3], a[3], kx[3], kv[3];
+    for (int d = 0; d < 7; ++d) c[d] = c0[d];
+    for (int d = 0; d < 3; ++d) {
+        v[d] = Yc[3 + d];
+        a[d] = cm_acc[d];
+        kx[d] = sc[d];
+        kv[d] = sc[3 + d];
+    }
+    for (int d = 0; d < 3; ++d) {
+        if (s == 0) v[d] = c[3 + d];
+        kx[d] = s == 0 ? v[d] : kx[d] + w * v[d];
+        kv[d] = s == 0 ? a[d] : kv[d] + w * a[d];
+    }
+    if (s < 3) {
         for (int d = 0; d < 3; ++d) {
-            kx[d] = s == 0 ? cs[3 + d] : sc[d] + w * cs[3 + d];
-            kv[d] = s == 0 ? cm_acc[d] : sc[3 + d] + w * cm_acc[d];
+            sc[d] = kx[d];
+            sc[3 + d] = kv[d];
+            out[d] = c[d] + h * v[d];
+            out[3 + d] = c[3 + d] + h * a[d];
         }
-        if (s < 3) {
-            for (int d = 0; d < 3; ++d) {
-                sc[d] = kx[d];
-                sc[3 + d] = kv[d];
-                const double v = cs[3 + d];
-                Ycn[d] = c0[d] + h * v;
-                Ycn[3 + d] = c0[3 + d] + h * cm_acc[d];
-            }
-            Ycn[6] = c0[6];
-            Ycn[7] = c0[7];
-        } else {
-            const double f = dt / 6.0;
-            for (int d = 0; d < 3; ++d) {
-                c0[d] += f * kx[d];
-                c0[3 + d] += f * kv[d];
-            }
+        out[6] = c[6];
+        out[7] = c0[7];
+    } else {
+        const double f = dt / 6.0;
+        for (int d = 0; d < 3; ++d) {
+            c0[d] = c[d] + f * kx[d];
+            c0[3 + d] = c[3 + d] + f * kv[d];
         }
     }
 }
@@ -130,12 +146,16 @@ __global__ __launch_bounds__(NT) void k_rk4_stage(int s, double dt, int n,
 }  // namespace
 
 ncg_status ncg_rk4_stage_launch(ncg_ctx *ctx, int s, double dt, int32_t n, const int32_t *ex,
-                                DBody *y0, const DBody *Y, DBody *Yn, const double *acc, double *sx,
-                                double *sv, double *c0, const double *Yc, double *Ycn,
-                                const double *cm, double *sc, hipStream_t st)
+                                DBody *y0, DBody *Y, DBody *Yn, const double *acc, double *sx,
+                                double *sv, double *c0, double *Yc, double *Ycn, const double *cm,
+                                double *sc, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_rk4_stage, dim3(cdiv(n, NT)), dim3(NT), 0, st, s, dt, (int)n, ex, y0, Y, Yn,
-                       acc, sx, sv, c0, Yc, Ycn, cm, sc);
+    if (Yn == Y)
+        hipLaunchKernelGGL(k_rk4_stage<true>, dim3(cdiv(n, NT)), dim3(NT), 0, st, s, dt, (int)n, ex,
+                           y0, Y, (DBody *)nullptr, acc, sx, sv, c0, Yc, (double *)nullptr, cm, sc);
+    else
+        hipLaunchKernelGGL(k_rk4_stage<false>, dim3(cdiv(n, NT)), dim3(NT), 0, st, s, dt, (int)n, ex,
+                           y0, Y, Yn, acc, sx, sv, c0, Yc, Ycn, cm, sc);
     NCG_CHECK_LAUNCH();
     return NCG_OK;
 }
@@ -162,9 +182,8 @@ static ncg_status rk4_body(ncg_ctx *ctx, DBody *y0, int32_t n, const int32_t *ex
                                       central_present ? dc : nullptr, G, soft, prec, acc, nullptr,
                                       central_present ? cm : nullptr, st);
         if (r != NCG_OK) return r;
-        hipLaunchKernelGGL(k_rk4_stage, dim3(cdiv(n, NT)), dim3(NT), 0, st, s, dt, (int)n, ex, y0, Y,
-                           Y, acc, sx, sv, c0, Yc, Yc, cm, sc);
-        NCG_CHECK_LAUNCH();
+        r = ncg_rk4_stage_launch(ctx, s, dt, n, ex, y0, Y, Y, acc, sx, sv, c0, Yc, Yc, cm, sc, st);
+        if (r != NCG_OK) return r;
     }
     return NCG_OK;
 }
