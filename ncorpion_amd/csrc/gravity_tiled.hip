@@ -11,7 +11,7 @@
 // 1 to 3, with Hilbert keys).
 //
 // Pipeline of one evaluation (all on one stream, no host synchronisation):
-//   1. k_bbox_*      bounding box, largest radius and mass, count of existing
+//   1. k_bbox_*      bounding box, largest radius (and mass), count of existing
 //                    bodies
 //   2. k_morton      mixed form: 30-bit Morton key per body over the bounding
 //                    CUBE (the same cell size on every axis, so that runs of
@@ -65,8 +65,11 @@ constexpr int NT = 256;     // threads per workgroup
 constexpr int BBP = 9;      // doubles of one partial of the bounding box
 
 // ---- 1. bounding box / count ---------------------------------------------
+// mass: the largest |mass| and the box's exponent too (the mixed form by unordered
+// pairs scales with them; the other forms' calls would pay 1.5 us of 140 at 8200
+// bodies for it).
 __global__ __launch_bounds__(NT) void k_bbox_partial(const DBody *__restrict__ b, int n,
-                                                     const int32_t *__restrict__ ex,
+                                                     const int32_t *__restrict__ ex, int mass,
                                                      double *__restrict__ part)
 {
     __shared__ double sh[NT];
@@ -80,7 +83,7 @@ __global__ __launch_bounds__(NT) void k_bbox_partial(const DBody *__restrict__ b
             mx[c] = fmax(mx[c], p[c]);
         }
         rm = fmax(rm, b[k].radius);
-        mm = fmax(mm, fabs(b[k].mass));
+        if (mass) mm = fmax(mm, fabs(b[k].mass));
         cnt += 1.0;
     }
     double *o = part + BBP * blockIdx.x;
@@ -94,12 +97,13 @@ __global__ __launch_bounds__(NT) void k_bbox_partial(const DBody *__restrict__ b
     if (threadIdx.x == 0) o[6] = v;
     v = block_reduce(cnt, sh, 2);
     if (threadIdx.x == 0) o[7] = v;
+    if (!mass) return;
     v = block_reduce(mm, sh, 1);
     if (threadIdx.x == 0) o[8] = v;
 }
 
 __global__ __launch_bounds__(NT) void k_bbox_final(const double *__restrict__ part, int nparts,
-                                                   Scal *__restrict__ sc)
+                                                   int mass, Scal *__restrict__ sc)
 {
     __shared__ double sh[NT];
     double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300}, rm = 0.0, cnt = 0.0;
@@ -112,7 +116,7 @@ __global__ __launch_bounds__(NT) void k_bbox_final(const double *__restrict__ pa
         }
         rm = fmax(rm, o[6]);
         cnt += o[7];
-        mm = fmax(mm, o[8]);
+        if (mass) mm = fmax(mm, o[8]);
     }
     double w = 0.0;
     for (int c = 0; c < 3; ++c) {
@@ -123,12 +127,15 @@ __global__ __launch_bounds__(NT) void k_bbox_final(const double *__restrict__ pa
             sc->bmax[c] = hi;
         }
     }
-    const double r = block_reduce(rm, sh, 1), m = block_reduce(mm, sh, 1);
-    const double nv = block_reduce(cnt, sh, 2);
+    const double r = block_reduce(rm, sh, 1), nv = block_reduce(cnt, sh, 2);
     if (threadIdx.x == 0) {
         sc->rmax = r;
-        sc->mmax = m;
         sc->nvalid = (int)nv;
+    }
+    if (!mass) return;
+    const double m = block_reduce(mm, sh, 1);
+    if (threadIdx.x == 0) {
+        sc->mmax = m;
         sc->lexp = exp_of(w);
     }
 }
@@ -754,8 +761,9 @@ static ncg_status tiled_order_w(ncg_ctx *ctx, const TiledShape &t, const TiledWo
 {
     // 2: along a Hilbert curve, for the mixed form by unordered pairs.
     const int spatial = prec == NCG_MIXED ? (mixed_sym_form(ctx, n, prec) ? 2 : 1) : 0;
-    hipLaunchKernelGGL(k_bbox_partial, dim3(t.nbb), dim3(NT), 0, st, d_b, n, d_ex, w.bpart);
-    hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(NT), 0, st, w.bpart, t.nbb, w.sc);
+    const int mass = spatial == 2;
+    hipLaunchKernelGGL(k_bbox_partial, dim3(t.nbb), dim3(NT), 0, st, d_b, n, d_ex, mass, w.bpart);
+    hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(NT), 0, st, w.bpart, t.nbb, mass, w.sc);
     hipLaunchKernelGGL(k_morton, dim3(cdiv(n, NT)), dim3(NT), 0, st, d_b, n, d_ex, w.sc, spatial,
                        w.key, w.idx);
     NCG_CHECK_LAUNCH();

@@ -24,9 +24,11 @@ struct TileHdr {
 
 struct Scal {           // per-evaluation scalars produced on the device
     double bmin[3], bmax[3];
-    double rmax, mmax;  // largest radius, largest |mass|
+    double rmax;        // largest radius
     int nvalid;
+    // Of an order along the Hilbert curve (the mixed form by unordered pairs):
     int lexp;           // exponent of the box's longest edge
+    double mmax;        // largest |mass|
 };
 
 // Powers of two that the mixed form by unordered pairs scales with: positions
