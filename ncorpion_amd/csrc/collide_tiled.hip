@@ -50,7 +50,8 @@ struct alignas(64) CpRec {
 };
 
 // Boxes of the tiles, one array of `ntiles` values per bound: positions lo
-// and hi, velocities lo and hi (three each), largest radius.
+// and hi, velocities lo and hi (three each), largest |radius| (the predicate
+// takes the square of a sum of radii, of any sign).
 constexpr int CBOX = 13;
 
 __device__ inline double wave_min(double v)
@@ -265,7 +266,7 @@ __global__ __launch_bounds__(CT) void k_cp_boxes(const CpRec *__restrict__ rec,
     const int nv = *nvalid;
     if (t >= ntiles || t * CPT >= nv) return;
     const CpRec r = rec[min(t * CPT + lane, nv - 1)];
-    const double v[7] = {r.x, r.y, r.z, r.vx, r.vy, r.vz, r.R};
+    const double v[7] = {r.x, r.y, r.z, r.vx, r.vy, r.vz, fabs(r.R)};
     double o[CBOX];
     for (int c = 0; c < 3; ++c) {
         o[c] = wave_min(v[c]);
@@ -320,7 +321,7 @@ __device__ inline CpBox body_box(const double *v /* x, y, z, vx, vy, vz, R */)
         o.lo[c] = o.hi[c] = v[c];
         o.vlo[c] = o.vhi[c] = v[3 + c];
     }
-    o.rmax = v[6];
+    o.rmax = fabs(v[6]);
     return o;
 }
 

@@ -69,7 +69,7 @@ struct CollHdr {
     double vx, vy, vz;     // velocity box centre
     float phx, phy, phz;   // half extents, rounded up
     float vhx, vhy, vhz;
-    float rmax;            // largest radius, rounded up
+    float rmax;            // largest |radius|, rounded up
     int count;
 };
 
@@ -536,7 +536,7 @@ __global__ __launch_bounds__(ENT) void k_ens_ctiles(const DBody *__restrict__ b,
             jc[s] = q;
             const double v[6] = {q.x, q.y, q.z, q.vx, q.vy, q.vz};
             for (int c = 0; c < 6; ++c) mn[r][c] = mx[r][c] = v[c];
-            rm[r] = q.radius;
+            rm[r] = fabs(q.radius);
         }
     }
     double cg[2][6], ct[6];
@@ -604,7 +604,7 @@ __device__ inline bool may_meet(const CollHdr &g, const CollHdr &t, double adt)
     return !(gx * gx + gy * gy + gz * gz > reach * reach);
 }
 
-// The header of a body alone (its radius rounded up).
+// The header of a body alone (its |radius| rounded up).
 __device__ inline CollHdr body_hdr(const DBody &q)
 {
     CollHdr h;
@@ -615,8 +615,8 @@ __device__ inline CollHdr body_hdr(const DBody &q)
     h.vy = q.vy;
     h.vz = q.vz;
     h.phx = h.phy = h.phz = h.vhx = h.vhy = h.vhz = 0.f;
-    float r = (float)q.radius;
-    if ((double)r < q.radius) r = nextafterf(r, 3.0e38f);
+    float r = fabsf((float)q.radius);
+    if ((double)r < fabs(q.radius)) r = nextafterf(r, 3.0e38f);
     h.rmax = r;
     h.count = 1;
     return h;

@@ -190,6 +190,24 @@ def test_replay_with_removed_and_created_bodies(ctx, seed):
     assert kinds == {0, 1, 2} and ref.largest >= n0  # removals, reuse and appends happened
 
 
+# The predicate takes the square of a sum of radii: a body with a negative one
+# meets those that a positive one of its size would.
+def test_tiled_pass_with_negative_radii(ctx):
+    import torch
+    from ncorpion_amd import ic
+    n, dt = 8200, 0.02
+    b = ic.disk(n, seed=3, mass=1e-8, radius=5e-4)
+    b[::40, 7] = -0.02
+    want, _, pairs = orc.brute_force(b, dt, 1, 1.5, 0, None)
+    assert len(pairs) > 50
+    want[:, 0:3] += dt * want[:, 3:6]
+    bt = torch.from_numpy(b).cuda()
+    ct = torch.zeros(8, dtype=torch.float64, device="cuda")
+    got = ctx.leapfrog_dev(bt, ct, 1, dt, 0.0, 0.0, "fast64", 1.5, 0, None, None)
+    assert got == len(pairs)
+    assert np.array_equal(bits(bt.cpu().numpy()), bits(want))
+
+
 # The tiled pass takes 8192 bodies and more; one body in the last tile, the
 # finer cells above 16,384, holes, a body whose radius reaches every tile, and
 # a replay that runs out of room (replayed on the host).

@@ -309,6 +309,18 @@ def _collision_run(ctx, systems, dt, steps, f=1.5):
     return nc, total
 
 
+def test_ensemble_collisions_with_negative_radii(ctx):
+    """The predicate takes the square of a sum of radii: a body with a negative
+    one meets those that a positive one of its size would."""
+    systems = []
+    for s, n in enumerate((65, 257, 385, 600)):
+        b = ic.disk(n, seed=800 + s, mass=1e-9, radius=1e-3)
+        b[::17, 7] = -0.03
+        systems.append(b)
+    nc, total = _collision_run(ctx, systems, 0.02, 1)
+    assert nc == total and total > 10, (nc, total)
+
+
 def test_ensemble_collisions_on_spread_disks_match_oracle(ctx):
     """Disks of 300-4000 bodies (the benchmark's kind, with R = 1e-3 for 42
     collisions): the collision pass tests only the tiles a group's position
