@@ -449,13 +449,14 @@ __global__ __launch_bounds__(SY_T, 4) void k_pairs_mix(const double4 *__restrict
 {
     __shared__ double4 rec[SY_C];
     __shared__ double js[3][SY_C];
-    if (!*far) return;  // no two groups are far: nothing to form or to add
     int r, c;
     sym_place(S, blockIdx.x, r, c);
     const int nv = scal->nvalid, tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j0 = c * SY_C, row0 = r * S.W, h0 = j0 / MG;
-    if (j0 >= nv || row0 >= nv) return;
+    // Without two far groups there is nothing to form or to add (the flag's load
+    // is one latency with nv's: before the others it cost 1.6 % at 65,536 bodies).
+    if (!*far || j0 >= nv || row0 >= nv) return;
 #pragma unroll
     for (int h = 0; h < SY_NB; ++h) {
         const int k = h * SY_T + tid;
