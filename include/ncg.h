@@ -190,8 +190,9 @@ ncg_status ncg_gravity_allpairs_dev(ncg_ctx *ctx, const ncg_body *d_bodies, int3
  * until the process ends; n above NCG_STATIC_MAX_N is refused
  * (NCG_ERR_INVALID).  The caller passes inputs and outputs as for
  * ncg_gravity_allpairs_dev, with the same results: NCG_F64_EXACT bit for bit;
- * the fast forms alike up to the grouping of the j-split sums (the split
- * count is lowered when the partials would not fit).  Every call on one GPU
+ * the fast forms alike up to FP64 rounding (every ordered pair is formed here,
+ * also where ncg_gravity_allpairs_dev forms unordered ones, and the split count
+ * is lowered when the partials would not fit).  Every call on one GPU
  * shares that GPU's array: calls that overlap on one GPU (from several
  * streams or threads) race.  Nothing is carried from one call to the next. */
 #define NCG_STATIC_SCRATCH_BYTES (32 << 20)
@@ -666,10 +667,11 @@ ncg_status ncg_cart2ell(ncg_ctx *ctx, const ncg_body *bodies, int32_t n, const i
  * per lane (1, 2, 4; 0 keeps), j-splits per i-block (0 = from the CU count,
  * -1 keeps), near/far threshold theta (<= 0 keeps), tile source (0 scalar
  * loads, 1 LDS, -1 keeps).  Results do not depend on the shape beyond FP
- * rounding of the split sums.  A shape set here selects the kernel it shapes
- * (every ordered pair); without one, NCG_F64_FAST of 4097 to 262144 bodies and
- * NCG_MIXED of NCG_STATIC_MAX_N + 1 to 262144 form each unordered pair once.  The
- * autotuner (ncorpion_amd/autotune.py) picks these per N.
+ * rounding of the split sums.  A shape (any of the three integers, other than
+ * "keep") selects the kernel it shapes (every ordered pair); without one,
+ * NCG_F64_FAST of 4097 to 262144 bodies and NCG_MIXED of NCG_STATIC_MAX_N + 1 to
+ * 262144 form each unordered pair once.  theta alone keeps that choice and applies
+ * to either kernel.  The autotuner (ncorpion_amd/autotune.py) picks these per N.
  */
 ncg_status ncg_set_tiling(ncg_ctx *ctx, int32_t ipl, int32_t nsplit, double theta, int32_t source);
 

@@ -615,6 +615,7 @@ extern "C" ncg_status ncg_set_tiling(ncg_ctx *ctx, int32_t ipl, int32_t nsplit, 
     NCG_REQUIRE(source >= -1 && source <= 1, "source must be 0 (scalar), 1 (LDS) or -1 (keep)");
     TiledCfg &c = ctx->tiled;
     ctx->tiled_explicit = true;
+    if (ipl > 0 || nsplit >= 0 || source >= 0) ctx->tiled_shaped = true;
     if (ipl > 0) c.ipl = ipl;
     if (nsplit >= 0) c.nsplit = nsplit;
     if (theta > 0.0) c.theta = theta;
@@ -749,7 +750,7 @@ static ncg_status work_eval_ctx(ncg_ctx *ctx, const TiledShape &t, int32_t n, bo
 // kernel, 0.50 by unordered pairs; of 262,144: 19.2 and 16.1.
 static bool mixed_sym_form(const ncg_ctx *ctx, int32_t n, ncg_precision prec)
 {
-    return prec == NCG_MIXED && n > NCG_STATIC_MAX_N && n <= NCG_SYM_MAX && !ctx->tiled_explicit;
+    return prec == NCG_MIXED && n > NCG_STATIC_MAX_N && n <= NCG_SYM_MAX && !ctx->tiled_shaped;
 }
 
 // The order of the evaluations that follow: spatial (Morton or Hilbert keys over
@@ -780,7 +781,7 @@ static ncg_status tiled_order_w(ncg_ctx *ctx, const TiledShape &t, const TiledWo
 // bodies 46 us against 112, 50,021 1.35 ms against 1.87, 200,000 17.8 against 24).
 static bool sym_form(const ncg_ctx *ctx, int32_t n, ncg_precision prec)
 {
-    return prec == NCG_F64_FAST && n > SMALL_N && n <= NCG_SYM_MAX && !ctx->tiled_explicit;
+    return prec == NCG_F64_FAST && n > SMALL_N && n <= NCG_SYM_MAX && !ctx->tiled_shaped;
 }
 
 ncg_status ncg_tiled_order(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int32_t *d_ex,

@@ -104,6 +104,7 @@ struct ncg_ctx {
     MeshState mesh;
     TiledCfg tiled;
     bool tiled_explicit = false;     // ncg_set_tiling overrides the table
+    bool tiled_shaped = false;       // it set a launch shape, not theta alone
     std::vector<TuneRow> tune;       // from the tuning table, sorted by n_min
     int num_cus = 0;
     bool profiling = false;

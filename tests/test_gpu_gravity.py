@@ -366,6 +366,34 @@ def test_mixed_pairs_match_fp64(ctx, n, soft, odd):
     assert np.all(none == 7.0)
 
 
+# theta set alone keeps the kernel (and its bits: the same theta from a table); a
+# launch shape selects the split kernel.
+@pytest.mark.parametrize("n,prec", [(5000, "fast64"), (33000, "mixed")])
+def test_theta_alone_keeps_the_unordered_form(monkeypatch, tmp_path, n, prec):
+    import torch
+    from ncorpion_amd import Context
+    table = tmp_path / "tuning.txt"
+    table.write_text("mixed 1 1 0 0.45 0\nfast64 1 1 0 0.45 0\n")
+    monkeypatch.setenv("NCG_TUNING", str(table))
+    m, R = ic.disk_c3_masses(n, n)
+    bt = torch.from_numpy(ic.disk(n, seed=n, masses=m, radii=R)).cuda()
+    got = []
+    for args in (None, dict(theta=0.45), dict(ipl=1, theta=0.45)):
+        ctx = Context(0)
+        try:
+            if args:
+                ctx.set_tiling(**args)
+            acc = torch.zeros((n, 3), dtype=torch.float64, device="cuda")
+            torch.cuda.synchronize()
+            ctx.gravity_allpairs_dev(bt, acc, None, None, 1.0, 0.0, prec)
+            ctx.synchronize()
+            got.append(acc.cpu().numpy())
+        finally:
+            ctx.close()
+    assert np.array_equal(bits(got[0]), bits(got[1]))
+    assert not np.array_equal(bits(got[0]), bits(got[2]))
+
+
 # Softening beyond the system: every pair of groups is near, the far kernel forms
 # nothing and its sums (an earlier call's) are left out.  FP64 sums of 3e4 terms:
 # ~sqrt(n) ulps, 1e-13.
