@@ -487,11 +487,12 @@ static ncg_status vjp_impl(ncg_ctx *ctx, const DBody *b, int32_t n, const double
     double *jv = dbuf<double>(ctx, "v_jv", 8 * (size_t)n);
     if (!gm_tmp || !part || !jv) return NCG_ERR_NOMEM;
     hipLaunchKernelGGL(k_vjp_pack, dim3(nb), dim3(AT), 0, st, b, (int)n, lam, soft, jv);
-    if (n >= VJP_SYM_MIN && n <= VJP_SYM_MAX) {
-        const SymShape S = sym_shape(n, 1, VI, n <= 32768 ? 4 : 8);
-        double *pi = dbuf<double>(ctx, "v_pi", 4 * (size_t)S.islots());
-        double *pj = dbuf<double>(ctx, "v_pj", 4 * (size_t)S.jslots());
-        if (!pi || !pj) return NCG_ERR_NOMEM;
+    const SymShape S = sym_shape(n, 1, VI, n <= 32768 ? 4 : 8);
+    if (n >= VJP_SYM_MIN && n <= VJP_SYM_MAX &&
+        ncg_pair_scratch(ctx, "v_pi", 32 * (size_t)S.islots(), "v_pj", 32 * (size_t)S.jslots(),
+                         true)) {
+        double *pi = static_cast<double *>(ctx->bufs["v_pi"].ptr);
+        double *pj = static_cast<double *>(ctx->bufs["v_pj"].ptr);
         ProfScope ps(ctx, st, "vjp");
         hipLaunchKernelGGL(k_vjp_sym, dim3((unsigned)S.workgroups()), dim3(SY_T), 0, st,
                            reinterpret_cast<const VjpRec *>(jv), S, pi, pj);

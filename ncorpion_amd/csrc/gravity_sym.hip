@@ -586,15 +586,32 @@ __global__ __launch_bounds__(FT) void k_sym_cm(const double *__restrict__ part, 
 // with 1, 2, 4; at 50,021 1.66, 1.46, 1.35).
 static int sym_reps(int32_t n) { return n <= 20000 ? 2 : n <= 65536 ? 4 : n <= 131072 ? 8 : 16; }
 
+static SymShape fast64_shape(int32_t n) { return sym_shape(n, SY_NB, GI, sym_reps(n)); }
+
+// Rows a row group: few where workgroups are few (32,800 bodies, 2 / 8: 0.44
+// and 0.50 ms), many where the partial sums weigh (262,144: 17.8 and 16.9).
+static SymShape mixed_shape(int32_t n)
+{
+    return sym_shape(n, SY_NB, MI, n <= 65536 ? 2 : n <= 131072 ? 4 : 8);
+}
+
+bool ncg_sym_room(ncg_ctx *ctx, int32_t n, ncg_precision prec, bool make)
+{
+    const SymShape S = prec == NCG_MIXED ? mixed_shape(n) : fast64_shape(n);
+    return ncg_pair_scratch(ctx, "y_pi", 24 * (size_t)S.islots(), "y_pj", 24 * (size_t)S.jslots(),
+                            make);
+}
+
+// Callers have ncg_sym_room's word for the partial sums.
 ncg_status ncg_gravity_sym(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int *d_perm,
                            const int *d_nvalid, const ncg_central *c, const double *d_central,
                            double G, double soft, double *d_acc, double *d_cm_acc, hipStream_t st)
 {
-    const SymShape S = sym_shape(n, SY_NB, GI, sym_reps(n));
+    const SymShape S = fast64_shape(n);
     double4 *jd = dbuf<double4>(ctx, "y_jd", n);
     double *jsig = dbuf<double>(ctx, "y_jsig", n);
-    double *pi = dbuf<double>(ctx, "y_pi", 3 * (size_t)S.islots());
-    double *pj = dbuf<double>(ctx, "y_pj", 3 * (size_t)S.jslots());
+    double *pi = static_cast<double *>(ctx->bufs["y_pi"].ptr);
+    double *pj = static_cast<double *>(ctx->bufs["y_pj"].ptr);
     const int nb = (int)cdiv(n, FS);
     double *cmpart = d_cm_acc ? dbuf<double>(ctx, "y_cm", 3 * (size_t)nb) : nullptr;
     if (!jd || !jsig || !pi || !pj || (d_cm_acc && !cmpart)) return NCG_ERR_NOMEM;
@@ -629,9 +646,7 @@ ncg_status ncg_gravity_mixed_sym(ncg_ctx *ctx, const DBody *d_b, int32_t n, cons
                                  double *d_cm_acc, hipStream_t st)
 {
     const Scal *scal = static_cast<const Scal *>(d_scal);
-    // Rows a row group: few where workgroups are few (32,800 bodies, 2 / 8: 0.44
-    // and 0.50 ms), many where the partial sums weigh (262,144: 17.8 and 16.9).
-    const SymShape S = sym_shape(n, SY_NB, MI, n <= 65536 ? 2 : n <= 131072 ? 4 : 8);
+    const SymShape S = mixed_shape(n);
     const int ng = (int)cdiv(n, MG), nw = (int)cdiv(ng, 64);
     double4 *jd = dbuf<double4>(ctx, "y_jd", (size_t)ng * MG);
     double *jsig = dbuf<double>(ctx, "y_jsig", (size_t)ng * MG);
@@ -639,8 +654,8 @@ ncg_status ncg_gravity_mixed_sym(ncg_ctx *ctx, const DBody *d_b, int32_t n, cons
     unsigned long long *mask = dbuf<unsigned long long>(ctx, "y_mask", (size_t)ng * nw);
     double *near = dbuf<double>(ctx, "y_near", 3 * (size_t)MNEAR * n);
     int *far = dbuf<int>(ctx, "y_far", 1);
-    double *pi = dbuf<double>(ctx, "y_pi", 3 * (size_t)S.islots());
-    double *pj = dbuf<double>(ctx, "y_pj", 3 * (size_t)S.jslots());
+    double *pi = static_cast<double *>(ctx->bufs["y_pi"].ptr);
+    double *pj = static_cast<double *>(ctx->bufs["y_pj"].ptr);
     const int nb = (int)cdiv(n, FS);
     double *cmpart = d_cm_acc ? dbuf<double>(ctx, "y_cm", 3 * (size_t)nb) : nullptr;
     if (!jd || !jsig || !hdr || !mask || !near || !far || !pi || !pj || (d_cm_acc && !cmpart))

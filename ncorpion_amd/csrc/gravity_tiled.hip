@@ -747,10 +747,13 @@ static ncg_status work_eval_ctx(ncg_ctx *ctx, const TiledShape &t, int32_t n, bo
 // partial sums and whose results are this one's up to the grouping of sums; up
 // to NCG_SYM_MAX bodies (partial sums of 1.6 GB); in a launch shape of the
 // caller's the split kernel runs.  Calls of 32,800 bodies: 0.57 ms with the split
-// kernel, 0.50 by unordered pairs; of 262,144: 19.2 and 16.1.
-static bool mixed_sym_form(const ncg_ctx *ctx, int32_t n, ncg_precision prec)
+// kernel, 0.50 by unordered pairs; of 262,144: 19.2 and 16.1.  make: the order is
+// formed, and the partial sums' buffers with it (the split kernel runs where they
+// cannot be).
+static bool mixed_sym_form(ncg_ctx *ctx, int32_t n, ncg_precision prec, bool make)
 {
-    return prec == NCG_MIXED && n > NCG_STATIC_MAX_N && n <= NCG_SYM_MAX && !ctx->tiled_shaped;
+    return prec == NCG_MIXED && n > NCG_STATIC_MAX_N && n <= NCG_SYM_MAX && !ctx->tiled_shaped &&
+           ncg_sym_room(ctx, n, prec, make);
 }
 
 // The order of the evaluations that follow: spatial (Morton or Hilbert keys over
@@ -761,7 +764,7 @@ static ncg_status tiled_order_w(ncg_ctx *ctx, const TiledShape &t, const TiledWo
                                 ncg_precision prec, hipStream_t st)
 {
     // 2: along a Hilbert curve, for the mixed form by unordered pairs.
-    const int spatial = prec == NCG_MIXED ? (mixed_sym_form(ctx, n, prec) ? 2 : 1) : 0;
+    const int spatial = prec == NCG_MIXED ? (mixed_sym_form(ctx, n, prec, true) ? 2 : 1) : 0;
     const int mass = spatial == 2;
     hipLaunchKernelGGL(k_bbox_partial, dim3(t.nbb), dim3(NT), 0, st, d_b, n, d_ex, mass, w.bpart);
     hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(NT), 0, st, w.bpart, t.nbb, mass, w.sc);
@@ -779,16 +782,17 @@ static ncg_status tiled_order_w(ncg_ctx *ctx, const TiledShape &t, const TiledWo
 // shape, and above NCG_SYM_MAX bodies the partial sums of the unordered form
 // would take more than 3.3 GB.  Faster at every size between (calls of 4200
 // bodies 46 us against 112, 50,021 1.35 ms against 1.87, 200,000 17.8 against 24).
-static bool sym_form(const ncg_ctx *ctx, int32_t n, ncg_precision prec)
+static bool sym_form(ncg_ctx *ctx, int32_t n, ncg_precision prec, bool make)
 {
-    return prec == NCG_F64_FAST && n > SMALL_N && n <= NCG_SYM_MAX && !ctx->tiled_shaped;
+    return prec == NCG_F64_FAST && n > SMALL_N && n <= NCG_SYM_MAX && !ctx->tiled_shaped &&
+           ncg_sym_room(ctx, n, prec, make);
 }
 
 ncg_status ncg_tiled_order(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int32_t *d_ex,
                            ncg_precision prec, hipStream_t st)
 {
     if (n <= SMALL_N) return NCG_OK;  // the direct form needs no order
-    if (sym_form(ctx, n, prec) && !d_ex) return NCG_OK;  // body order
+    if (sym_form(ctx, n, prec, true) && !d_ex) return NCG_OK;  // body order
     const TiledShape t = tiled_shape(ctx, n, NCG_MIXED);
     TiledWork w;
     ncg_status r = work_order_ctx(ctx, t, n, st, w);
@@ -894,7 +898,7 @@ ncg_status ncg_tiled_eval(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int32
         return ncg_small_launch(ctx, d_b, n, d_ex, c, d_central, G, soft, d_acc, cterm, p3,
                                 d_cm_acc, st);
     }
-    if (sym_form(ctx, n, prec)) {
+    if (sym_form(ctx, n, prec, false)) {
         const int *perm = nullptr, *nvalid = nullptr;
         if (d_ex) {  // the order of ncg_tiled_order: existing bodies first
             perm = dbuf<int>(ctx, "t_perm", n);
@@ -904,7 +908,7 @@ ncg_status ncg_tiled_eval(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int32
         }
         return ncg_gravity_sym(ctx, d_b, n, perm, nvalid, c, d_central, G, soft, d_acc, d_cm_acc, st);
     }
-    if (mixed_sym_form(ctx, n, prec)) {
+    if (mixed_sym_form(ctx, n, prec, false)) {
         const int *perm = dbuf<int>(ctx, "t_perm", n);
         const Scal *sc = dbuf<Scal>(ctx, "t_scal", 1);
         if (!perm || !sc) return NCG_ERR_NOMEM;

@@ -21,19 +21,57 @@ ncg_status ncg_fail(ncg_ctx *ctx, ncg_status code, const char *fmt, ...)
     return code;
 }
 
+void ncg_dbuf_release(ncg_ctx *ctx, const char *name)
+{
+    DevBuf &b = ctx->bufs[name];
+    if (!b.ptr) return;
+    // The old contents may still be read by queued work on the stream.
+    (void)hipStreamSynchronize(ctx->stream);
+    (void)hipFree(b.ptr);
+    b.ptr = nullptr;
+    b.bytes = 0;
+    ctx->buf_gen++;  // captured graphs hold the address
+}
+
+bool ncg_pair_scratch(ncg_ctx *ctx, const char *name1, size_t bytes1, const char *name2,
+                      size_t bytes2, bool make)
+{
+    if (ctx->pair_scratch > 0 && bytes1 + bytes2 > ctx->pair_scratch) return false;
+    const char *name[2] = {name1, name2};
+    const size_t bytes[2] = {bytes1, bytes2};
+    for (int k = 0; k < 2; ++k) {
+        DevBuf &b = ctx->bufs[name[k]];
+        if (b.ptr && b.bytes >= bytes[k]) continue;
+        if (!make || ctx->capturing) return false;
+        ncg_dbuf_release(ctx, name[k]);
+        // With room to grow, else to size.
+        for (size_t want : {bytes[k] + bytes[k] / 4, bytes[k]}) {
+            if (hipMalloc(&b.ptr, want) == hipSuccess) {
+                b.bytes = want;
+                ctx->buf_gen++;
+                break;
+            }
+            (void)hipGetLastError();  // not the next launch's error
+            b.ptr = nullptr;
+        }
+        if (!b.ptr) {
+            ncg_dbuf_release(ctx, name1);  // leaves what there is to the other form
+            return false;
+        }
+    }
+    return true;
+}
+
 void *ncg_dbuf(ncg_ctx *ctx, const char *name, size_t bytes)
 {
     DevBuf &b = ctx->bufs[name];
     if (b.bytes >= bytes && b.ptr) return b.ptr;
     if (b.ptr) {
-        // The old contents may still be read by queued work on the stream.
-        (void)hipStreamSynchronize(ctx->stream);
-        (void)hipFree(b.ptr);
-        b.ptr = nullptr;
-        b.bytes = 0;
+        ncg_dbuf_release(ctx, name);
     }
     size_t want = bytes + bytes / 4 + 256;
     if (hipMalloc(&b.ptr, want) != hipSuccess) {
+        (void)hipGetLastError();  // not the next launch's error
         b.ptr = nullptr;
         ncg_fail(ctx, NCG_ERR_NOMEM, "hipMalloc of %zu bytes for '%s' failed", want, name);
         return nullptr;
@@ -147,6 +185,10 @@ ncg_status ncg_create(ncg_ctx **out, int device)
     if (const char *rc = getenv("NCG_REPLAY_CAP")) {
         const long v = atol(rc);
         if (v > 0 && v < (1L << 30)) ctx->replay_cap = (unsigned)v;
+    }
+    if (const char *ps = getenv("NCG_PAIR_SCRATCH")) {
+        const long long v = atoll(ps);
+        if (v > 0) ctx->pair_scratch = (size_t)v;
     }
     if (const char *cd = getenv("NCG_REPLAY_CLUSTER_DIST")) {
         const long v = atol(cd);

@@ -116,6 +116,9 @@ struct ncg_ctx {
     // loops); NCG_REPLAY_CAP in the environment lowers it (tests of the
     // overflow fallback).  0 = each loop's default.
     unsigned replay_cap = 0;
+    // Bytes of partial sums that the pair forms by unordered pairs may hold at
+    // most (NCG_PAIR_SCRATCH in the environment; 0 = what can be allocated).
+    size_t pair_scratch = 0;
     // Cells between visits of one cluster of the parallel mesh replay
     // (NCG_REPLAY_CLUSTER_DIST; a test knob: 0 makes clusters meet).
     int replay_cluster_dist = 4;
@@ -243,6 +246,14 @@ ncg_status ncg_fail(ncg_ctx *ctx, ncg_status code, const char *fmt, ...);
 // Device scratch buffer `name`, grown to at least `bytes` (contents are not
 // preserved across growth).  Returns nullptr and records an error on failure.
 void *ncg_dbuf(ncg_ctx *ctx, const char *name, size_t bytes);
+void ncg_dbuf_release(ncg_ctx *ctx, const char *name);
+
+// Whether the two buffers of partial sums of a form by unordered pairs, which grow
+// as n^2, are there: made if they can be (make; never during a capture).  False,
+// without an error, leaves the call to the form by ordered pairs, which needs
+// less.
+bool ncg_pair_scratch(ncg_ctx *ctx, const char *name1, size_t bytes1, const char *name2,
+                      size_t bytes2, bool make);
 
 template <class T>
 static inline T *dbuf(ncg_ctx *ctx, const char *name, size_t count)
@@ -323,6 +334,8 @@ ncg_status ncg_gravity_dev_impl(ncg_ctx *ctx, const DBody *d_bodies, int32_t n,
 // (slots to bodies; null: body order) and d_nvalid (existing bodies; null: n).
 // d_central: the central body in a device record; else c (may be null).
 constexpr int NCG_SYM_MAX = 262144;
+// Whether the partial sums of n bodies' form are there (ncg_pair_scratch).
+bool ncg_sym_room(ncg_ctx *ctx, int32_t n, ncg_precision prec, bool make);
 ncg_status ncg_gravity_sym(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int *d_perm,
                            const int *d_nvalid, const ncg_central *c, const double *d_central,
                            double G, double soft, double *d_acc, double *d_cm_acc, hipStream_t st);

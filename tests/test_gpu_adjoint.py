@@ -289,6 +289,34 @@ def test_checkpointed_forward_and_backward_match_all_in_one(ctx):
         assert float((u - w).abs().max()) <= 1e-13 * scale
 
 
+# Without room for its partial sums the ordered pairs run (FP64 sums of 1e4
+# terms: 1e-12 normwise).
+def test_vjp_without_room_for_partial_sums(monkeypatch):
+    torch = tt()
+    from ncorpion_amd import Context
+    n = 10300
+    b = torch.from_numpy(disk(n, n)).cuda()
+    lam = torch.from_numpy(np.random.default_rng(n).normal(size=(n, 3))).cuda()
+    cen = torch.tensor([0, 0, 0, 0, 0, 0, 1.0, 1.0], dtype=torch.float64, device="cuda")
+    got = []
+    for room in ("", "100000"):
+        monkeypatch.setenv("NCG_PAIR_SCRATCH", room)
+        ctx = Context(0)
+        try:
+            gx = torch.zeros((n, 3), dtype=torch.float64, device="cuda")
+            gm = torch.zeros(n, dtype=torch.float64, device="cuda")
+            gc = torch.zeros(4, dtype=torch.float64, device="cuda")
+            torch.cuda.synchronize()
+            ctx.vjp_gravity_dev(b, cen, lam, gx, gm, gc, None, 1.0, 1.0)
+            ctx.synchronize()
+            got.append([t.clone() for t in (gx, gm, gc)])
+        finally:
+            ctx.close()
+    assert not torch.equal(got[0][0], got[1][0])
+    for a, r in zip(*got):
+        assert float((a - r).norm() / r.norm()) < 1e-12
+
+
 # The pair part by unordered pairs (10,240 to 131,072 bodies): chunks of 512
 # bodies, row groups of 64, or 128 above 32,768; both remainders.  Against the
 # dense formula; tolerance: sums of ~1e4 terms in FP64, 1e-12 normwise.

@@ -366,6 +366,45 @@ def test_mixed_pairs_match_fp64(ctx, n, soft, odd):
     assert np.all(none == 7.0)
 
 
+# Without room for the partial sums of the unordered forms (here a bound of the
+# caller's; an allocation that fails takes the same path) the ordered forms run:
+# fields with and without holes, and graphs of RK4 steps, whose capture must not
+# allocate.  FP64 sums of 1e4 terms: 1e-13; mixed against FP64 as above.
+@pytest.mark.parametrize("n,prec", [(5000, "fast64"), (33000, "mixed")])
+def test_fields_without_room_for_partial_sums(monkeypatch, n, prec):
+    import torch
+    from ncorpion_amd import Context
+    m, R = ic.disk_c3_masses(n, n)
+    bt = torch.from_numpy(ic.disk(n, seed=n, masses=m, radii=R)).cuda()
+    et = torch.from_numpy((np.arange(n) % 11 != 3).astype(np.int32)).cuda()
+    got = {}
+    for room in ("", "100000"):
+        monkeypatch.setenv("NCG_PAIR_SCRATCH", room)
+        ctx = Context(0)
+        try:
+            for e in (None, et):
+                acc = torch.zeros((n, 3), dtype=torch.float64, device="cuda")
+                torch.cuda.synchronize()
+                ctx.gravity_allpairs_dev(bt, acc, e, None, 1.0, 0.0, prec)
+                ctx.synchronize()
+                got[room, e is None] = acc.cpu().numpy()
+            runs = []
+            for graph in (False, True):
+                x = bt.clone()
+                c = torch.tensor([0, 0, 0, 0, 0, 0, 1.0, 1.0], dtype=torch.float64, device="cuda")
+                torch.cuda.synchronize()
+                ctx.rk4_steps_dev(x, c, 4, 0.01, 1.0, 0.0, prec, graph=graph)
+                ctx.synchronize()
+                runs.append(x.cpu().numpy())
+            assert np.array_equal(bits(runs[0]), bits(runs[1]))
+        finally:
+            ctx.close()
+    for whole in (True, False):
+        a, r = got["100000", whole], got["", whole]
+        assert not np.array_equal(bits(a), bits(r))
+        assert np.linalg.norm(a - r) < (1e-13 if prec == "fast64" else 1.5e-7) * np.linalg.norm(r)
+
+
 # theta set alone keeps the kernel (and its bits: the same theta from a table); a
 # launch shape selects the split kernel.
 @pytest.mark.parametrize("n,prec", [(5000, "fast64"), (33000, "mixed")])
