@@ -426,7 +426,7 @@ __global__ __launch_bounds__(64) void k_cp_pairs(const CpRec *__restrict__ rec,
 // ---- replay ------------------------------------------------------------------
 constexpr int RPT = 1024;     // threads of the replay
 constexpr int RP_EV = NCG_CP_EVENTS;
-constexpr int RP_DYN = 2048;  // pairs found by the scans of changed bodies
+constexpr int RP_DYN = NCG_CP_FOUND;
 constexpr int RP_CH = NCG_CP_CHANGED;
 
 __device__ inline unsigned long long pair_key(int a, int c)
@@ -441,8 +441,9 @@ __device__ inline unsigned long long pair_key(int a, int c)
 // take part in.  A pair is decided with the states it has when its turn comes
 // (NcorpiON's rule), and every pair that can be accepted then is listed: its
 // bodies' last changes were followed by a scan at those states.  did_collide
-// and holes as in k_bf_replay.  err: 1 more candidates than cap, 2 than RP_EV,
-// 4 more changed bodies or found pairs than fit; the state is then not valid.
+// and holes as in k_bf_replay.  err: 1 more candidates than cap, 2 than RP_EV
+// (both with nothing changed), 4 more changed bodies or found pairs than fit (in
+// the middle of the pass): the caller restores the state and replays on the host.
 __global__ __launch_bounds__(RPT) void k_cp_replay(
     DBody *__restrict__ b, const int32_t *__restrict__ ex, int32_t *__restrict__ dc, int one_coll,
     const CpRec *__restrict__ rec, const int *__restrict__ nvalid, int ntiles,
@@ -452,7 +453,7 @@ __global__ __launch_bounds__(RPT) void k_cp_replay(
 {
     __shared__ unsigned long long ev[RP_EV], dyn[RP_DYN];
     __shared__ int ch[RP_CH], tl[RPT];
-    __shared__ int s_nd, s_ndyn, s_nt, s_i, s_j;
+    __shared__ int s_nd, s_ndyn, s_nt, s_i, s_j, s_known;
     __shared__ unsigned long long s_cur;
     const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
     const unsigned long long total = *count;
@@ -534,6 +535,7 @@ __global__ __launch_bounds__(RPT) void k_cp_replay(
                 s_i = i;
                 s_j = j;
                 s_cur = cur;
+                s_known = 0;
             }
             __threadfence_block();
         }
@@ -584,19 +586,23 @@ __global__ __launch_bounds__(RPT) void k_cp_replay(
         const int nd = s_nd;
         for (int q = tid; q < nd; q += RPT) {
             const int o = ch[q];
+            if (o == i) atomicOr(&s_known, 1);
+            if (o == j) atomicOr(&s_known, 2);
             const DBody X = b[o];
             found(i, A, o, X.x, X.y, X.z, X.vx, X.vy, X.vz, X.radius);
             found(j, B, o, X.x, X.y, X.z, X.vx, X.vy, X.vz, X.radius);
         }
         __syncthreads();
-        if (s_ndyn > RP_DYN || nd + 2 > RP_CH) {
+        const int known = s_known;
+        if (s_ndyn > RP_DYN || nd + 2 - __popc(known) > RP_CH) {
             if (tid == 0) atomicOr(err, 4u);
             break;
         }
         if (tid == 0) {
-            ch[nd] = i;
-            ch[nd + 1] = j;
-            s_nd = nd + 2;
+            int m2 = nd;
+            if (!(known & 1)) ch[m2++] = i;
+            if (!(known & 2)) ch[m2++] = j;
+            s_nd = m2;
         }
         __syncthreads();
     }

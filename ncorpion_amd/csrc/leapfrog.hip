@@ -1168,10 +1168,12 @@ ncg_status leapfrog_run(ncg_ctx *ctx, ncg_body *d_bodies, int32_t n_in, int32_t 
     if (hs[1])
         return ncg_fail(ctx, NCG_ERR_CAPACITY,
                         "collision replay capacity exceeded (flags %u: 1 = more than %u candidates, "
-                        "2 = more than %d to decide, 4 = more than %d changed bodies in one pass); "
-                        "results are not valid",
+                        "2 = more than %d to decide, 4 = more than %d changed bodies in one pass, or "
+                        "from %d bodies more than %d pairs found after changes); results are not "
+                        "valid",
                         hs[1], cap, n >= NCG_CP_MIN ? NCG_CP_EVENTS : NCG_REPLAY_RCAP,
-                        n >= NCG_CP_MIN ? NCG_CP_CHANGED : NCG_REPLAY_DCAP);
+                        n >= NCG_CP_MIN ? NCG_CP_CHANGED : NCG_REPLAY_DCAP, NCG_CP_MIN,
+                        NCG_CP_FOUND);
     return NCG_OK;
 }
 

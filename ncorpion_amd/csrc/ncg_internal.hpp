@@ -181,7 +181,8 @@ ncg_status ncg_candidates_launch(ncg_ctx *ctx, const DBody *d_b, int32_t n, cons
 // more than they save).
 constexpr int NCG_CP_MIN = 8192;
 constexpr int NCG_CP_EVENTS = 4096;   // candidates of a pass the tiled replay takes
-constexpr int NCG_CP_CHANGED = 1024;  // bodies changed in a pass it takes
+constexpr int NCG_CP_CHANGED = 1024;  // bodies changed in a pass it takes (each once)
+constexpr int NCG_CP_FOUND = 2048;    // pairs that the scans of changed bodies may add
 ncg_status ncg_cp_candidates_launch(ncg_ctx *ctx, const DBody *d_b, int32_t n, const int32_t *d_ex,
                                     double dt, int2 *d_out, unsigned long long cap,
                                     unsigned long long *d_count, hipStream_t st);

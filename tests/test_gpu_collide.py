@@ -190,6 +190,38 @@ def test_replay_with_removed_and_created_bodies(ctx, seed):
     assert kinds == {0, 1, 2} and ref.largest >= n0  # removals, reuse and appends happened
 
 
+# The limits of the tiled replay: more than 4096 candidates; more than 1024 changed
+# bodies, and just fewer in more than 512 collisions; a clump whose changed bodies
+# have more than 2048 later pairs.  Past a limit the pass is undone and replayed on
+# the host; the results are the oracle's either way.
+@pytest.mark.parametrize("kind,radius", [("candidates", 0.035), ("changed", 0.014),
+                                         ("fewer", 0.0128), ("found", 1e-4)])
+def test_tiled_replay_limits(ctx, kind, radius):
+    import torch
+    n, dt = 8200, 0.02
+    rng = np.random.default_rng(n)
+    b = np.zeros((n, 8))
+    b[:, 0:3] = rng.uniform(-1, 1, (n, 3))
+    b[:, 3:6] = rng.normal(size=(n, 3))
+    b[:, 6], b[:, 7] = 1e-8, radius
+    if kind == "found":
+        b[:110, 0:3] = 5.0 + rng.uniform(-0.1, 0.1, (110, 3))
+        b[:110, 3:6] *= 3.0
+        b[:110, 7] = 0.08
+    want, _, pairs = orc.brute_force(b, dt, 1, 1.5, 0, None)
+    cand, changed = len(ctx.collide_candidates(b, None, dt)), len(set(pairs.ravel()))
+    assert (cand > 4096) == (kind == "candidates")
+    assert (changed > 1024) == (kind in ("candidates", "changed"))
+    assert len(pairs) > (512 if kind != "found" else 300)
+    want[:, 0:3] += dt * want[:, 3:6]
+    bt = torch.from_numpy(b).cuda()
+    ct = torch.zeros(8, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    got = ctx.leapfrog_dev(bt, ct, 1, dt, 0.0, 0.0, "fast64", 1.5, 0, None, None)
+    assert got == len(pairs)
+    assert np.array_equal(bits(bt.cpu().numpy()), bits(want))
+
+
 # The predicate takes the square of a sum of radii: a body with a negative one
 # meets those that a positive one of its size would.
 def test_tiled_pass_with_negative_radii(ctx):
