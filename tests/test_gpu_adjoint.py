@@ -289,6 +289,34 @@ def test_checkpointed_forward_and_backward_match_all_in_one(ctx):
         assert float((u - w).abs().max()) <= 1e-13 * scale
 
 
+# Both sides of the unordered pairs' upper end (131,072 bodies), at the edges of
+# chunks and row groups: rows of the dense formula; sums of ~1e5 terms in FP64, 1e-12.
+@pytest.mark.parametrize("n", [131072, 131073])
+def test_vjp_rows_at_the_largest_unordered_form(ctx, n):
+    torch = tt()
+    b = torch.from_numpy(disk(n, 7)).cuda()
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    lam = torch.randn((n, 3), generator=gen, dtype=torch.float64, device="cuda")
+    cen = torch.zeros(8, dtype=torch.float64, device="cuda")
+    gx = torch.zeros((n, 3), dtype=torch.float64, device="cuda")
+    gm = torch.zeros(n, dtype=torch.float64, device="cuda")
+    gc = torch.zeros(4, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    ctx.vjp_gravity_dev(b, cen, lam, gx, gm, gc, None, 1.0, 1.0)
+    ctx.synchronize()
+    x, m, R = b[:, 0:3], b[:, 6], b[:, 7]
+    rows = torch.tensor([0, 1, 127, 128, 511, 512, 65535, 65536, n - 513, n - 2, n - 1], device="cuda")
+    d = x[None, :, :] - x[rows, None, :]
+    D2 = (d * d).sum(-1) + (R[rows, None] + R[None, :]) ** 2
+    i3 = D2 ** -1.5
+    i3[torch.arange(len(rows)), rows] = 0.0
+    u = m[rows, None, None] * lam[None] - m[None, :, None] * lam[rows, None, :]
+    rx = (u * i3[..., None] - 3.0 * d * ((d * u).sum(-1) * i3 / D2)[..., None]).sum(1)
+    rm = -((lam[None] * d).sum(-1) * i3).sum(1)
+    assert float((gx[rows] - rx).norm() / rx.norm()) < 1e-12
+    assert float((gm[rows] - rm).norm() / rm.norm()) < 1e-12
+
+
 # Without room for its partial sums the ordered pairs run (FP64 sums of 1e4
 # terms: 1e-12 normwise).
 def test_vjp_without_room_for_partial_sums(monkeypatch):

@@ -366,6 +366,31 @@ def test_mixed_pairs_match_fp64(ctx, n, soft, odd):
     assert np.all(none == 7.0)
 
 
+# The largest row groups (512 slots from 131,073 bodies in FP64-fast, 1024 in mixed)
+# and both sides of the unordered forms' upper end (262,144): rows at every edge of
+# chunks and row groups, with holes, against the oracle's sums (FP64: ~sqrt(n) ulps
+# of a sum whose terms partly cancel, 1e-12; mixed: a term's FP32 rounding, 2^-24 (1 +
+# 2 / theta) = 4.6e-7 at theta 0.3, twice over for a body whose terms cancel).
+@pytest.mark.parametrize("n", [131073, 262144, 262145])
+@pytest.mark.parametrize("prec,tol", [("fast64", 1e-12), ("mixed", 1e-6)])
+def test_unordered_forms_at_their_largest(ctx, n, prec, tol):
+    import torch
+    m, R = ic.disk_c3_masses(n, n)
+    b = ic.disk(n, seed=n, masses=m, radii=R)
+    ex = (np.random.default_rng(n).uniform(size=n) > 0.07).astype(np.int32)
+    rows = np.array([0, 511, 512, 1023, 1024, 65535, 131071, 131072, n - 1023, n - 2, n - 1])
+    ex[rows] = 1
+    bt = torch.from_numpy(b).cuda()
+    for e in (None, ex):
+        acc = torch.zeros((n, 3), dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        et = None if e is None else torch.from_numpy(e).cuda()
+        ctx.gravity_allpairs_dev(bt, acc, et, None, 1.0, 1e-6, prec)
+        ctx.synchronize()
+        ref = orc.vector_field_rows(b, rows, e, None, 1.0, 1e-6)
+        assert rel_err(acc.cpu().numpy()[rows], ref)[0] < tol
+
+
 # Without room for the partial sums of the unordered forms (here a bound of the
 # caller's; an allocation that fails takes the same path) the ordered forms run:
 # fields with and without holes, and graphs of RK4 steps, whose capture must not
