@@ -1,12 +1,14 @@
 """Autotuner of the gravity launch shapes.
 
-Single systems (the split pair kernel; its theta also serves the mixed form by
-unordered pairs): for each body count N (a seeded disk of that size), every
-candidate shape -- bodies per lane, j-splits per i-block, tile source (scalar
-loads or LDS) and, for the mixed form, the near/far threshold theta -- is
-timed with HIP events around the pair kernel.  A theta is admissible only if
-the mixed form's max relative error on the mutual acceleration, against the
-FP64 form, stays below `max_err`.
+Single systems: for each body count N (a seeded disk of that size), every
+candidate shape of the split pair kernel -- bodies per lane, j-splits per
+i-block, tile source (scalar loads or LDS) and, for the mixed form, the near/far
+threshold theta -- is timed with HIP events around the pair kernel.  A theta is
+admissible only if the max relative error on the mutual acceleration of the
+mixed form that runs at N, against the FP64 form, stays below `max_err`.  Where
+that is the form by unordered pairs (32,769 to 262,144 bodies), theta is the
+fastest admissible one of that form, and the shapes (which run without room for its
+partial sums) are timed with it.
 
 Ensembles: on 512 seeded disks of log-uniform N in [256, 8192], bodies per
 lane of the FP64-fast ensemble pass are timed the same way, and the mixed
@@ -16,7 +18,7 @@ The fastest admissible shape per (form, N) is written to the tuning table
 that libncg.so reads at context creation (ncg_tuning.txt beside it); rows of
 forms that were not tuned are kept.
 
-    python -m ncorpion_amd.autotune --n 8192 16384 65536 262144 \
+    python -m ncorpion_amd.autotune --n 8192 32768 49152 131072 262144 294912 \
         --out ncorpion_amd/ncg_tuning.txt
 
 Sizes up to 4096 are skipped (the direct form serves them); the first tuned
@@ -34,6 +36,9 @@ DEFAULT_TABLE = os.path.join(HERE, "ncg_tuning.txt")
 # Up to this many bodies the fast forms run the direct kernel (k_small), which
 # has no tiled launch shape: every candidate would time the same.
 DIRECT_MAX_N = 4096
+# Bodies for which the mixed form runs by unordered pairs (ncg_set_tiling in ncg.h);
+# fewer and more run the split kernel.
+UNORDERED_N = range(32769, 262145)
 
 
 def _workload(n, seed=0):
@@ -55,22 +60,42 @@ def _time(ctx, bt, acc, prec, reps, soft):
     return ms / max(cnt, 1)
 
 
-def tune(ctx, n, reps=3, max_err=5e-7, soft=1e-6, thetas=(0.3, 0.35, 0.5), log=print):
+def mixed_errors(bt, thetas, soft, reps):
+    """{theta: (max relative error, ms)} of the mixed form that runs by default
+    for these bodies (a context of its own: a launch shape set in another would
+    select the split kernel)."""
+    import torch
+    from . import Context
+    acc = torch.zeros((bt.shape[0], 3), dtype=torch.float64, device="cuda")
+    ref = torch.zeros_like(acc)
+    ctx = Context(0)
+    try:
+        ctx.gravity_allpairs_dev(bt, ref, None, None, 1.0, soft, "fast64")
+        ctx.synchronize()
+        rnorm = torch.linalg.norm(ref, dim=1)
+        out = {}
+        for theta in thetas:
+            ctx.set_tiling(theta=theta)
+            ms = _time(ctx, bt, acc, "mixed", reps, soft)
+            out[theta] = (float(torch.max(torch.linalg.norm(acc - ref, dim=1) / rnorm)), ms)
+    finally:
+        ctx.close()
+    return out
+
+
+def tune(ctx, n, reps=3, max_err=5e-7, soft=1e-6, thetas=(0.3, 0.35, 0.4, 0.5), log=print):
     """Returns {form: (ipl, nsplit, theta, src, ms)} for N = n.  When no
     theta keeps the mixed form within max_err, the most accurate one is
     used (and said so).  The thetas start at 0.3: a far pair's FP32
     separation error is at most u (1 + 2/theta) relative (u = 2^-24), 4.6e-7
     there, and smaller thetas, admissible on one tuning disk, were not on
-    others."""
+    others.  (The largest relative error is that of a body whose mutual
+    acceleration nearly cancels, |a| some 1e-3 of the rms: other disks of 2e5
+    bodies and more reach 1e-6 to 2e-6 in either form at these thetas.)"""
     import torch
     b = _workload(n)
     bt = torch.from_numpy(b).cuda()
     acc = torch.zeros((n, 3), dtype=torch.float64, device="cuda")
-    ref = torch.zeros_like(acc)
-    ctx.set_tiling(1, 0, 0.35, 0)
-    ctx.gravity_allpairs_dev(bt, ref, None, None, 1.0, soft, "fast64")
-    ctx.synchronize()
-    rnorm = torch.linalg.norm(ref, dim=1)
     cus = 256
     nib1 = max(1, -(-n // 256))
     splits = sorted({s for s in (1, 2, 4, 8, 16, 32, 64, 128, 256, 512) if s * nib1 <= 512 * cus})
@@ -79,18 +104,16 @@ def tune(ctx, n, reps=3, max_err=5e-7, soft=1e-6, thetas=(0.3, 0.35, 0.5), log=p
         best = None
         cands = (0.35,)
         if prec == "mixed":
-            errs = {}
+            errs = mixed_errors(bt, thetas, soft, reps)
             for theta in thetas:
-                ctx.set_tiling(1, 0, theta, 0)
-                ctx.gravity_allpairs_dev(bt, acc, None, None, 1.0, soft, "mixed")
-                ctx.synchronize()
-                errs[theta] = float(torch.max(torch.linalg.norm(acc - ref, dim=1) / rnorm))
-                log("  n=%d theta=%.2f max rel err %.2e" % (n, theta, errs[theta]))
-            cands = tuple(t for t in thetas if errs[t] <= max_err)
+                log("  n=%d theta=%.2f max rel err %.3e, %.3f ms" % ((n, theta) + errs[theta]))
+            cands = tuple(t for t in thetas if errs[t][0] <= max_err)
             if not cands:
                 cands = (min(errs, key=errs.get),)
                 log("  n=%d: no theta within %.1e; using the most accurate, %.2f" %
                     (n, max_err, cands[0]))
+            elif n in UNORDERED_N:
+                cands = (min(cands, key=lambda t: errs[t][1]),)
         timed = []
         for theta in cands:
             for ipl, src, ns in itertools.product((1, 2), (0, 1), splits):
@@ -100,6 +123,8 @@ def tune(ctx, n, reps=3, max_err=5e-7, soft=1e-6, thetas=(0.3, 0.35, 0.5), log=p
         # j-splits: each split writes (and the finish reads) 24 B per body.
         fastest = min(t[4] for t in timed)
         best = min((t for t in timed if t[4] <= 1.01 * fastest), key=lambda t: (t[1], t[4]))
+        if prec == "mixed" and n in UNORDERED_N:
+            best = best[:4] + (errs[best[2]][1],)  # the time of the form that runs
         out[prec] = best
         log("  n=%d %s best ipl=%d nsplit=%d theta=%.2f src=%d %.3f ms" % ((n, prec) + best))
     return out
@@ -195,7 +220,7 @@ def write_table(rows, path):
 
 def main(argv=None):
     ap = argparse.ArgumentParser(description=__doc__.split("\n")[0])
-    ap.add_argument("--n", type=int, nargs="+", default=[8192, 16384, 65536, 262144])
+    ap.add_argument("--n", type=int, nargs="+", default=[8192, 32768, 49152, 131072, 262144, 294912])
     ap.add_argument("--out", default=DEFAULT_TABLE)
     ap.add_argument("--max-err", type=float, default=5e-7)
     ap.add_argument("--json", default=None)
@@ -218,8 +243,12 @@ def main(argv=None):
         for i, n in enumerate(ns):
             r = tune(ctx, n, max_err=args.max_err, log=log)
             res[n] = r
-            # A row applies from the geometric midpoint to the previous size.
+            # A row applies from the geometric midpoint to the previous size,
+            # or from where the mixed form changes between the two.
             nmin = 1 if i == 0 else int((ns[i - 1] * n) ** 0.5)
+            for edge in (UNORDERED_N.start, UNORDERED_N.stop):
+                if i > 0 and ns[i - 1] < edge <= n:
+                    nmin = edge
             for prec in ("mixed", "fast64"):
                 if r[prec] is not None:
                     rows.append((prec, nmin, r[prec]))

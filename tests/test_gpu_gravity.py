@@ -430,6 +430,25 @@ def test_fields_without_room_for_partial_sums(monkeypatch, n, prec):
         assert np.linalg.norm(a - r) < (1e-13 if prec == "fast64" else 1.5e-7) * np.linalg.norm(r)
 
 
+# The tuning table's bound on the largest relative error (5e-7), on the disks that
+# the tuner measures and the kernels that run at their sizes.
+@pytest.mark.parametrize("n", [32768, 49152, 131072, 262144])
+def test_mixed_error_within_the_tuners_bound(n):
+    import torch
+    from ncorpion_amd import Context, autotune
+    bt = torch.from_numpy(autotune._workload(n)).cuda()
+    acc = {p: torch.zeros((n, 3), dtype=torch.float64, device="cuda") for p in ("mixed", "fast64")}
+    ctx = Context(0)
+    try:
+        torch.cuda.synchronize()
+        for p, a in acc.items():
+            ctx.gravity_allpairs_dev(bt, a, None, None, 1.0, 1e-6, p)
+        ctx.synchronize()
+    finally:
+        ctx.close()
+    assert rel_err(acc["mixed"].cpu().numpy(), acc["fast64"].cpu().numpy())[0] <= 5e-7
+
+
 # theta set alone keeps the kernel (and its bits: the same theta from a table); a
 # launch shape selects the split kernel.
 @pytest.mark.parametrize("n,prec", [(5000, "fast64"), (33000, "mixed")])
