@@ -114,11 +114,20 @@ def traffic_run(n, timeout=150):
     return out
 
 
+def unordered_pairs(n):
+    """Whether the mixed form runs by unordered pairs (ncg_set_tiling in ncg.h)."""
+    return 32768 < n <= 262144
+
+
 def pairs_algorithmic_bytes(n):
-    """Bytes the pair kernel must move per launch: the sorted FP64 records
-    (32 B) and softening lengths (8 B) read once, 24 B of acceleration partials
-    written per body."""
-    return n * (32 + 8 + 24)
+    """Bytes the pair kernels must move per launch: the sorted FP64 records
+    (32 B) and softening lengths (8 B), and the split kernel's FP32 far-form
+    records (16 B), read once, 24 B of accelerations written per body.  The
+    measured traffic is more: partial sums (at 262,144 bodies 1.7 GB written by
+    unordered pairs, 0.8 GB by the split kernel's 128 splits), and by unordered
+    pairs a chunk's records read by each of its workgroups (1.1 GB) and spilled
+    registers."""
+    return n * (32 + 8 + (0 if unordered_pairs(n) else 16) + 24)
 
 
 def make_workload(n, seed=0):
@@ -834,10 +843,13 @@ def main():
                      "peak": PEAK_FP32_VECTOR_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved_tflops / PEAK_FP32_VECTOR_TFLOPS,
                      "traffic": None,
-                     "kernel": "k_mix_near + k_pairs_mix" if 32768 < n <= 262144
+                     "kernel": "k_mix_near + k_pairs_mix" if unordered_pairs(n)
                      else "k_pairs<mixed>", "kernel_avg_ms": kavg_ms,
                      "kernel_launches": nl_mix,
-                     "flop_per_interaction": FLOP_PER_INTERACTION},
+                     "flop_per_interaction": FLOP_PER_INTERACTION,
+                     "note": "20 flop for each ordered interaction; by unordered pairs the two "
+                             "of a pair share their separation and 1/r^3, so fewer are executed"
+                     if unordered_pairs(n) else "20 flop for each ordered interaction"},
     }
 
     if not args.no_traffic:

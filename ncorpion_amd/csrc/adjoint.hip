@@ -139,9 +139,10 @@ __global__ __launch_bounds__(AT) void k_vjp_reduce(const double4 *__restrict__ p
 // The pair part by unordered pairs (sym_dev.hpp): with u = m_i lam_j - m_j
 // lam_i, the pair adds T u to g_x_i and -T u to g_x_j, -G lam_j . d / D^3 to
 // g_m_i and G lam_i . d / D^3 to g_m_j: 47 FP64 instructions and one v_rsq_f64 a
-// pair, against 38 and one for each of the two.  16,384 bodies: 276 us (382 by
-// ordered pairs); four bodies i a wavefront spilled (1320 us), with fewer
-// wavefronts a SIMD 384.
+// pair, against 38 and one for each of the two: 56 VALU instructions issued a
+// wavefront of pairs, in 328 clocks a SIMD (counters at 16,384 bodies).  16,384
+// bodies: 275 to 281 us (382 by ordered pairs); four bodies i a wavefront spilled
+// (1320 us), with fewer wavefronts a SIMD 384.
 constexpr int VI = 2;    // bodies i of a wavefront
 constexpr int VROW = SY_WAVES * VI;
 
@@ -464,8 +465,8 @@ __global__ void k_adj_zero(double *__restrict__ a, int n)
 
 // Bodies for which the pair part runs by unordered pairs: 114 us against 112 by
 // ordered ones at 8192 bodies (too few workgroups), 57 against 37 at 4096, 364
-// against 438 at 16,384 with the sums; above 131,072 the partial sums take more
-// than 4 GB.
+// against 438 at 16,384 with the sums; above 131,072 the partial sums, which grow as
+// n^2, take more than 2.7 GB.
 static constexpr int VJP_SYM_MIN = 10240, VJP_SYM_MAX = 131072;
 
 // VJP at body state b (positions and masses) with central state cen (8):

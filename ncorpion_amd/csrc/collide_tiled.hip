@@ -5,8 +5,8 @@
 // pair i < j is a candidate exactly when closest_approach's predicate accepts
 // it (collide_allpairs.hip tests all of them), but a pair can only meet within
 // dt when its distance is at most R + |dv| |dt|.  The bodies are put into the
-// cells of a Morton grid by a counting sort, cut into tiles of 64, and a tile
-// pair whose boxes (of positions, of velocities, and the largest radius) are
+// cells of a Hilbert grid by a counting sort, cut into tiles of 64, and a tile
+// pair whose boxes (of positions, of velocities, and the largest |radius|) are
 // farther apart than that is skipped, then each body of a tile pair left that
 // is too far from the other tile's box.  What remains is tested with the same
 // predicate, so the candidates are the same set whatever the order of the
@@ -621,8 +621,8 @@ struct CpWork {
 
 ncg_status cp_work(ncg_ctx *ctx, int32_t n, CpWork &w)
 {
-    // Cells of about a tile's bodies on a thin disk: 64 cells an axis up to
-    // 131,072 bodies (1.1e3 of them hold a disk around the origin), 128 above.
+    // Cells smaller than a tile on a thin disk: 64 cells an axis up to 16,384
+    // bodies (some 1.1e3 of them hold a disk around the origin), 128 above.
     w.bits = n <= (1 << 14) ? 6 : 7;
     w.bins = 1 << (3 * w.bits);
     w.nblk = w.bins / CBIN;

@@ -102,6 +102,7 @@ __device__ inline void box_axis(double lo, double hi, double &c, float &h)
 }
 
 // ---- order ------------------------------------------------------------------
+// One workgroup per system: bounding cube, largest radius, and the keys
 // (system << 30) | Hilbert index over the cube.
 __global__ __launch_bounds__(ENT) void k_ens_keys(const DBody *__restrict__ b,
                                                   const EnsSys *__restrict__ sys,

@@ -5,8 +5,9 @@
 // In the reference, body k starts from the central term, subtracts
 // G*m_p*(X_k-X_p)/D^3 for p < k while k is the outer body, and later receives
 // += G*m_q*(X_q-X_k)/D^3 from every q > k as they become the outer body.  For
-// body k that is one sequential sum over j ascending, j != k.  One lane owns
-// one body and walks j in that order through LDS tiles; the p < k terms are
+// body k that is one sequential sum over j ascending, j != k.  A workgroup holds
+// four bodies: lanes of three wavefronts form the terms, one j each, and one lane
+// per component of the fourth adds them in that order; the p < k terms are
 // formed exactly as the reference forms them (X_k - X_p, then subtracted) and
 // the q > k terms likewise (X_q - X_k, then added), so signed zeros match too.
 // This translation unit is compiled with -ffp-contract=off: no FMA fusion.
@@ -49,13 +50,15 @@ __device__ inline void exact_term(double X, double Y, double Z, double Rk, doubl
 // the same way from the per-body reaction terms (physics.c:141-146 adds them
 // body by body), beside the other blocks.
 //
-// What bounds it: below ~5000 bodies the chain of dependent additions (5.7
-// clocks each), above it the FP64 issue of the terms (44 instructions when the
-// operands are in the window of exact_term.hpp).  EXP_B = 4 makes the two
-// halves of a chunk about equal (192 additions ~1100 clocks, 4 terms ~900).
+// What bounds it: from ~5000 bodies the FP64 issue of the terms (44 instructions
+// when the operands are in the window of exact_term.hpp).  Below that neither half
+// alone: at 2000 bodies the chain of dependent additions (5.7 clocks each) takes 5
+// us and the terms' issue about 7 of the kernel's 22; where the rest goes (start,
+// barriers of the 11 chunks, first loads) is not measured.  EXP_B = 4 makes the
+// two halves of a chunk about equal (192 additions ~1100 clocks, 4 terms ~900).
 // One wavefront per body, its three summing lanes idle during the terms and
 // the other 61 during the sums, took 40 us at 2000 bodies and 2.27 ms at 20,011
-// (and CM_acc 13 and 101 us after it); this form takes 24 us and 1.16 ms with
+// (and CM_acc 13 and 101 us after it); this form takes 22 us and 1.13 ms with
 // CM_acc.  One body per lane, the form above 32,768 bodies before, took 25.7 ms
 // at 65,536 and 212 ms at 262,144, this one 10.9 and 171.  EXP_B = 2 takes 1.66 ms
 // at 20,011 (the summing wavefronts' share), 8 (two workgroups a CU by LDS) 1.17.

@@ -5,11 +5,12 @@
 // with one separation, one 1/D and one D^-3 for both.  A pair is 22 FP64
 // instructions (20 without softening) and one v_rsq_f64 (17 clocks a wavefront,
 // as much as 3.5 others), where the split kernel takes 18 (16) and one v_rsq_f64
-// for each of the two: 123 against 206 clocks of issue, of which 165 are reached
-// (the rest: barriers, the j sums in LDS, the sums over lanes).  50,021 bodies:
-// 1.87 ms a call with the split kernel, 1.35 here; 100,003: 6.12 and 4.8; 16,384:
-// 0.32 and 0.19.  Eight bodies i a wavefront spilled or left two wavefronts a
-// SIMD (2.0 ms at 50,021); their records read from LDS bound it by LDS (1.44).
+// for each of the two: 123 against 206 clocks of issue a wavefront of pairs, which
+// takes 154 (counters at 50,021 bodies; the rest: 29 instructions issued in all,
+// barriers, the j sums in LDS, the sums over lanes).  50,021 bodies: 1.76 ms a call
+// with the split kernel, 1.30 here; 100,003: 6.4 and 5.0; 16,384: 0.28 and 0.17.
+// Eight bodies i a wavefront spilled or left two wavefronts a SIMD (2.0 ms at
+// 50,021); their records read from LDS bound it by LDS (1.44).
 #include <algorithm>
 
 #include "ncg_internal.hpp"
@@ -256,7 +257,8 @@ __global__ __launch_bounds__(FT) void k_sym_records(const DBody *__restrict__ b,
 //         taken from the box centre of i's group in FP64 and rounded once; 16
 //         instructions and a v_rsq_f32 a pair, where the scaled far term of the
 //         split kernel takes 11 and one for each of the two: 51 against 76
-//         clocks of issue a wavefront, of which 73 are reached (the rest: j
+//         clocks of issue a wavefront of pairs, which takes 67 at 262,144 bodies
+//         and 72 at 100,003 (counters; the rest: 19.5 instructions issued in all, j
 //         records and sums in LDS, barriers).  Operands are vector registers (a
 //         scalar one takes the issue from 2.6 to 4.4 clocks).
 // A lane's FP32 sums are 16 terms of a body j, or 16 of a body i, and i's over 8
@@ -264,9 +266,10 @@ __global__ __launch_bounds__(FT) void k_sym_records(const DBody *__restrict__ b,
 // (the box's edge and the largest G m about 1), so that no system of units over-
 // or underflows FP32 (the FP64 terms are unchanged by it, but for results at the
 // ends of its range).
-// Calls of 262,144 bodies: 19.2 ms with the split kernel, 16.1 here; 100,003:
-// 3.40 and 2.87; 32,800: 0.57 and 0.50; the field's error against FP64 is that
-// of the split kernel (4.9e-9 and 5.0e-9, 2.3e-9 and 2.2e-9, 1.8e-9 and 1.3e-9).
+// Calls of 262,144 bodies: 19.4 ms with the split kernel, 16.1 here; 100,003:
+// 3.17 and 2.66; 32,800: 0.49 and 0.42; the field's error against FP64 is that
+// of the split kernel or less (norm 2.3e-9 and 2.0e-9, 1.5e-9 and 1.5e-9, 1.6e-9
+// and 1.1e-9).
 // Eight bodies i a wavefront: 21.2 ms at 262,144 (the j records and sums come
 // twice as often); sums over all lanes in FP32: error +10 %.
 constexpr int MI = 16;            // bodies i of a wavefront

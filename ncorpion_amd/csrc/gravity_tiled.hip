@@ -746,8 +746,8 @@ static ncg_status work_eval_ctx(ncg_ctx *ctx, const TiledShape &t, int32_t n, bo
 // sizes of the allocation-free entry point, whose scratch cannot hold the
 // partial sums and whose results are this one's up to the grouping of sums; up
 // to NCG_SYM_MAX bodies (partial sums of 1.6 GB); in a launch shape of the
-// caller's the split kernel runs.  Calls of 32,800 bodies: 0.57 ms with the split
-// kernel, 0.50 by unordered pairs; of 262,144: 19.2 and 16.1.  make: the order is
+// caller's the split kernel runs.  Calls of 32,800 bodies: 0.49 ms with the split
+// kernel, 0.42 by unordered pairs; of 262,144: 19.4 and 16.1.  make: the order is
 // formed, and the partial sums' buffers with it (the split kernel runs where they
 // cannot be).
 static bool mixed_sym_form(ncg_ctx *ctx, int32_t n, ncg_precision prec, bool make)
@@ -780,8 +780,8 @@ static ncg_status tiled_order_w(ncg_ctx *ctx, const TiledShape &t, const TiledWo
 // Whether the FP64-fast form runs by unordered pairs (gravity_sym.hip): with a
 // launch shape of the caller's (ncg_set_tiling) the split kernel runs in that
 // shape, and above NCG_SYM_MAX bodies the partial sums of the unordered form
-// would take more than 3.3 GB.  Faster at every size between (calls of 4200
-// bodies 46 us against 112, 50,021 1.35 ms against 1.87, 200,000 17.8 against 24).
+// would take more than 2.4 GB.  Faster at every size between (calls of 4200
+// bodies 34 us against 93, 50,021 1.30 ms against 1.76, 200,000 19.8 against 25.1).
 static bool sym_form(ncg_ctx *ctx, int32_t n, ncg_precision prec, bool make)
 {
     return prec == NCG_F64_FAST && n > SMALL_N && n <= NCG_SYM_MAX && !ctx->tiled_shaped &&

@@ -83,7 +83,6 @@ __device__ inline unsigned hilbert(unsigned x, unsigned y, unsigned z)
     return (expand10(X[0]) << 2) | (expand10(X[1]) << 1) | expand10(X[2]);
 }
 
-// One workgroup per system: bounding cube, largest radius, and the keys
 template <class T>
 __device__ inline T block_reduce(T v, T *sh, int op /*0 min 1 max 2 sum*/)
 {
