@@ -52,10 +52,11 @@ __device__ inline void exact_term(double X, double Y, double Z, double Rk, doubl
 //
 // What bounds it: from ~5000 bodies the FP64 issue of the terms (44 instructions
 // when the operands are in the window of exact_term.hpp).  Below that neither half
-// alone: at 2000 bodies the chain of dependent additions (5.7 clocks each) takes 5
-// us and the terms' issue about 7 of the kernel's 22; where the rest goes (start,
-// barriers of the 11 chunks, first loads) is not measured.  EXP_B = 4 makes the
-// two halves of a chunk about equal (192 additions ~1100 clocks, 4 terms ~900).
+// alone: of 22 us at 2000 bodies the chain of dependent additions (5.7 clocks each)
+// takes 5 and the issue of the terms about 9 (85 instructions a wavefront of them);
+// a wavefront lives 40,000 clocks (counters), 16,000 of them waiting, with two
+// wavefronts a SIMD.  EXP_B = 4 makes the two halves of a chunk about equal (192
+// additions ~1100 clocks, 4 terms ~900).
 // One wavefront per body, its three summing lanes idle during the terms and
 // the other 61 during the sums, took 40 us at 2000 bodies and 2.27 ms at 20,011
 // (and CM_acc 13 and 101 us after it); this form takes 22 us and 1.13 ms with
