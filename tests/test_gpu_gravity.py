@@ -252,6 +252,28 @@ def test_exact_bitwise_edges(ctx, n, kind, soft):
         assert np.array_equal(bits(cm), bits(rcm))
 
 
+# Massless and negative bodies are in the window: their terms' zeros and signs.
+@pytest.mark.parametrize("n", [65, 193, 577])
+def test_exact_massless_and_negative_bodies(ctx, n):
+    b = _exact_edge_bodies(n, "planar")
+    b[::3, 6] = 0.0
+    b[1::6, 6] = -0.0
+    b[2::3, 6] *= -1.0
+    b[n // 2, 6] = 2.0 ** 100     # above the window
+    cen = (0.1, 0.2, 0.0, 1.0)
+    for soft in (0.0, 1e-3):
+        for c in (None, cen):
+            ref, rcm = orc.vector_field_brute(b, None, c, 1.0, soft)
+            acc, cm = ctx.gravity_allpairs(b, None, c, 1.0, soft, "exact")
+            assert np.all((bits(acc) == bits(ref)) | (np.isnan(acc) & np.isnan(ref)))
+            if c is not None:
+                assert np.array_equal(bits(cm), bits(rcm))
+    b[:, 6] = 0.0
+    ref, _ = orc.vector_field_brute(b, None, None, 1.0, 0.0)
+    acc, _ = ctx.gravity_allpairs(b, None, None, 1.0, 0.0, "exact")
+    assert np.array_equal(bits(acc), bits(ref))
+
+
 # A flat disk with both zeros on the axis and the central body in its plane: the
 # z sum of the last body at +0 is -0 (its central term, or start value, and
 # every term after it), which a term of +0 for one of -0 would turn.
