@@ -33,7 +33,7 @@ __device__ inline bool coord_ok(double v)
 }
 
 // G m zero or |G m| in [2^-100, 2^100).  (With massless and negative ones outside
-// the window, 1000 such bodies took 17.0 to 18.8 us, XXX so.)
+// the window, a field of 1000 such bodies took 17.0 to 19.0 us, 12.1 to 12.4 so.)
 __device__ inline bool gm_ok(double v)
 {
     return (hi_word(v) & 0x7fffffffu) - ((1023u - 100u) << 20) < (200u << 20) || v == 0.0;

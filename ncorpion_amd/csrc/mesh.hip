@@ -975,11 +975,15 @@ __global__ __launch_bounds__(MR_T) void k_mesh_replay(
 }
 
 // ---- neighbour-cell gravity ---------------------------------------------------
-// Term G m_p (X_p - X_k) / D^3 of physics.c:186-200 (reference expression).
+// Term of physics.c:186-200 (reference expression) for body k at (X, Y, Z): FST, k
+// is the pair's first (the visitor), - G m_p (X_k - X_p) / D^3; else + G m_p (X_p -
+// X_k) / D^3.  The two differ in the sign of a zero only.
+template <bool FST>
 __device__ inline void term_exact(double X, double Y, double Z, double Rk, double4 p, double Rp,
                                   double G, double s, double &ax, double &ay, double &az)
 {
-    const double dx = X - p.x, dy = Y - p.y, dz = Z - p.z;
+    const double dx = FST ? X - p.x : p.x - X, dy = FST ? Y - p.y : p.y - Y,
+                 dz = FST ? Z - p.z : p.z - Z;
     const double soft = s * (Rk + Rp);
     const double D = sqrt(dx * dx + dy * dy + dz * dz + soft * soft);
     const double D3 = D * D * D;
@@ -987,9 +991,9 @@ __device__ inline void term_exact(double X, double Y, double Z, double Rk, doubl
     {
         double q0, q1, q2;
         div3(gm * dx, gm * dy, gm * dz, D3, q0, q1, q2);
-        ax -= q0;
-        ay -= q1;
-        az -= q2;
+        ax = FST ? ax - q0 : ax + q0;
+        ay = FST ? ay - q1 : ay + q1;
+        az = FST ? az - q2 : az + q2;
     }
 }
 
@@ -1003,11 +1007,13 @@ __device__ inline bool term_ok(double x, double y, double z, double gm, double R
 // term_exact through the window form when every active lane's operands allow it
 // (kok, pok: the bodies' parts).  k_mord, 2^20 bodies: 4.73 ms with sqrt and
 // div3 in every term, 4.01 with this; 16,384 bodies 173 and 127 us.
+template <bool FST>
 __device__ inline void term_window(double X, double Y, double Z, double Rk, bool kok, double4 p,
                                    double Rp, bool pok, double G, double s, double &ax,
                                    double &ay, double &az)
 {
-    const double dx = X - p.x, dy = Y - p.y, dz = Z - p.z;
+    const double dx = FST ? X - p.x : p.x - X, dy = FST ? Y - p.y : p.y - Y,
+                 dz = FST ? Z - p.z : p.z - Z;
     double r2 = dx * dx + dy * dy + dz * dz;
     if (s != 0.0) {
         const double soft = s * (Rk + Rp);
@@ -1016,12 +1022,12 @@ __device__ inline void term_window(double X, double Y, double Z, double Rk, bool
     if (__all(kok && pok && r2_ok(r2))) {
         const double gm = G * p.w;
         double v[3] = {gm * dx, gm * dy, gm * dz};
-        window_quotients<true>(v, r2);
+        window_quotients<FST>(v, r2);
         ax += v[0];
         ay += v[1];
         az += v[2];
     } else {
-        term_exact(X, Y, Z, Rk, p, Rp, G, s, ax, ay, az);
+        term_exact<FST>(X, Y, Z, Rk, p, Rp, G, s, ax, ay, az);
     }
 }
 
@@ -1118,8 +1124,8 @@ __global__ __launch_bounds__(MT) void k_mgrav_rest(const DBody *__restrict__ b, 
         for (int big = 0; big < 3 && big < n; ++big) {
             if (ex && !ex[big]) continue;
             const DBody g = b[big];
-            term_exact(q.x, q.y, q.z, q.radius, make_double4(g.x, g.y, g.z, g.mass), g.radius, G, s,
-                       ax, ay, az);
+            term_exact<true>(q.x, q.y, q.z, q.radius, make_double4(g.x, g.y, g.z, g.mass), g.radius,
+                             G, s, ax, ay, az);
         }
     acc[3 * (size_t)k + 0] = ax;
     acc[3 * (size_t)k + 1] = ay;
@@ -1174,8 +1180,8 @@ __global__ __launch_bounds__(MT) void k_mgrav(const DBody *__restrict__ b, int n
     for (int big = 0; big < 3 && big < n; ++big) {
         if (ex && !ex[big]) continue;
         const DBody g = b[big];
-        term_exact(me.x, me.y, me.z, me.radius, make_double4(g.x, g.y, g.z, g.mass), g.radius, G,
-                   s, ax, ay, az);
+        term_exact<true>(me.x, me.y, me.z, me.radius, make_double4(g.x, g.y, g.z, g.mass), g.radius,
+                         G, s, ax, ay, az);
     }
     const long kk = skey[t];
     for (int r = 0; r < 9; ++r) {
@@ -1387,13 +1393,14 @@ __device__ inline bool bv_has(const int *__restrict__ o, int a, int e, int x)
 
 // Term of body v (by id) on the body at (X, Y, Z) of radius Rk; pairs with a
 // body 0..2 or an absent body are skipped as in physics.c:351.
+template <bool FST>
 __device__ inline void term_id(const DBody *__restrict__ b, const int32_t *__restrict__ ex, int v,
                                double X, double Y, double Z, double Rk, double G, double s,
                                double &ax, double &ay, double &az)
 {
     if (v <= 2 || (ex && !ex[v])) return;
     const DBody q = b[v];
-    term_exact(X, Y, Z, Rk, make_double4(q.x, q.y, q.z, q.mass), q.radius, G, s, ax, ay, az);
+    term_exact<FST>(X, Y, Z, Rk, make_double4(q.x, q.y, q.z, q.mass), q.radius, G, s, ax, ay, az);
 }
 
 // Next recorded big visit from index vi on that lists body k (NOKEY if none).
@@ -1520,14 +1527,14 @@ __global__ __launch_bounds__(MT) void k_mord(const DBody *__restrict__ b, int n,
     for (int big = 0; big < 3 && big < n; ++big) {
         if (ex && !ex[big]) continue;
         const DBody g = b[big];
-        term_exact(me.x, me.y, me.z, Rk, make_double4(g.x, g.y, g.z, g.mass), g.radius, G, s, ax,
-                   ay, az);
+        term_exact<true>(me.x, me.y, me.z, Rk, make_double4(g.x, g.y, g.z, g.mass), g.radius, G, s,
+                         ax, ay, az);
     }
     // (1) big visits before k.
     int vi = 0;
     for (; vi < nbv && bvk[vi] < k; ++vi)
         if (bvk[vi] > 2 && bv_has(bvo, bvoff[vi], bvoff[vi + 1], k))
-            term_id(b, ex, bvk[vi], me.x, me.y, me.z, Rk, G, s, ax, ay, az);
+            term_id<false>(b, ex, bvk[vi], me.x, me.y, me.z, Rk, G, s, ax, ay, az);
     // The lanes of one cell walk the same positions in step (so that their
     // loads coincide), each lane adding only the terms that are its own.
     const long kk = skey[t];
@@ -1560,7 +1567,7 @@ __global__ __launch_bounds__(MT) void k_mord(const DBody *__restrict__ b, int n,
                 nr = rr[u + 1];
             }
             if (idu < k && xu)
-                term_window(me.x, me.y, me.z, Rk, kok, pu, ru, (xu & 2) != 0, G, s, ax, ay, az);
+                term_window<true>(me.x, me.y, me.z, Rk, kok, pu, ru, (xu & 2) != 0, G, s, ax, ay, az);
         }
     }
     // (3) later visits: the cell's id-ordered neighbourhood list after k's own
@@ -1592,15 +1599,15 @@ __global__ __launch_bounds__(MT) void k_mord(const DBody *__restrict__ b, int n,
         if (nb != NOKEY) {
             const unsigned id = (unsigned)sid[u];
             while (nb < id) {
-                term_id(b, ex, (int)nb, me.x, me.y, me.z, Rk, G, s, ax, ay, az);
+                term_id<false>(b, ex, (int)nb, me.x, me.y, me.z, Rk, G, s, ax, ay, az);
                 ++vi;
                 nb = next_big(bvk, bvoff, bvo, nbv, vi, k);
             }
         }
-        if (xu) term_window(me.x, me.y, me.z, Rk, kok, pu, ru, (xu & 2) != 0, G, s, ax, ay, az);
+        if (xu) term_window<false>(me.x, me.y, me.z, Rk, kok, pu, ru, (xu & 2) != 0, G, s, ax, ay, az);
     }
     while (nb != NOKEY) {
-        term_id(b, ex, (int)nb, me.x, me.y, me.z, Rk, G, s, ax, ay, az);
+        term_id<false>(b, ex, (int)nb, me.x, me.y, me.z, Rk, G, s, ax, ay, az);
         ++vi;
         nb = next_big(bvk, bvoff, bvo, nbv, vi, k);
     }
@@ -1635,16 +1642,16 @@ __global__ __launch_bounds__(MT) void k_mrest_ord(const DBody *__restrict__ b, i
     for (int big = 0; big < 3; ++big) {
         if (ex && !ex[big]) continue;
         const DBody g = b[big];
-        term_exact(q.x, q.y, q.z, q.radius, make_double4(g.x, g.y, g.z, g.mass), g.radius, G, s, ax,
-                   ay, az);
+        term_exact<true>(q.x, q.y, q.z, q.radius, make_double4(g.x, g.y, g.z, g.mass), g.radius, G, s,
+                         ax, ay, az);
     }
     for (int vi = 0; vi < nbv; ++vi) {
         const int v = bvk[vi];
         if (v == k) {
             for (int u = bvoff[vi]; u < bvoff[vi + 1]; ++u)
-                term_id(b, ex, bvo[u], q.x, q.y, q.z, q.radius, G, s, ax, ay, az);
+                term_id<true>(b, ex, bvo[u], q.x, q.y, q.z, q.radius, G, s, ax, ay, az);
         } else if (v > 2 && bv_has(bvo, bvoff[vi], bvoff[vi + 1], k)) {
-            term_id(b, ex, v, q.x, q.y, q.z, q.radius, G, s, ax, ay, az);
+            term_id<false>(b, ex, v, q.x, q.y, q.z, q.radius, G, s, ax, ay, az);
         }
     }
     acc[3 * (size_t)k + 0] = ax;
@@ -1677,11 +1684,11 @@ __global__ __launch_bounds__(MT) void k_mexplicit(const DBody *__restrict__ b,
     for (int big = 0; big < 3; ++big) {
         if (ex && !ex[big]) continue;
         const DBody g = b[big];
-        term_exact(q.x, q.y, q.z, q.radius, make_double4(g.x, g.y, g.z, g.mass), g.radius, G, s, ax,
-                   ay, az);
+        term_exact<true>(q.x, q.y, q.z, q.radius, make_double4(g.x, g.y, g.z, g.mass), g.radius, G, s,
+                         ax, ay, az);
     }
     for (int u = first; u < first + cnt; ++u)
-        term_id(b, ex, pl[u], q.x, q.y, q.z, q.radius, G, s, ax, ay, az);
+        term_id<true>(b, ex, pl[u], q.x, q.y, q.z, q.radius, G, s, ax, ay, az);
     acc[3 * (size_t)k + 0] = ax;
     acc[3 * (size_t)k + 1] = ay;
     acc[3 * (size_t)k + 2] = az;

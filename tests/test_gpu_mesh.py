@@ -185,6 +185,28 @@ def test_mesh_gravity_exact_in_pair_list_order(ctx, seed, mode, nbig, holes, cen
         assert np.array_equal(bits(cm), bits(rcm))
 
 
+@pytest.mark.parametrize("n,both", [(600, False), (600, True), (3000, True)])
+def test_mesh_gravity_exact_keeps_the_sign_of_zero(ctx, n, both):
+    """A flat disk (z = 0 of one sign or both) about a central body in its plane,
+    with massless bodies: a pair's term has the sign that its first and its second
+    body give it (physics.c:186-200), which decides that of a zero sum."""
+    b = blob(n, 7, half=0.03)
+    b[:, 2] = b[:, 5] = 0.0
+    if both:
+        b[::3, 2] = -0.0
+    b[n // 4::5, 6] = 0.0
+    ex = np.ones(n, np.int32)
+    ctx.mesh_pass(b, ex, 0.0, 0.004, 0.128, 32, 1)
+    pairs = ctx.mesh_pairs()
+    for central in (None, (0.0, 0.0, 0.0, 1.0)):
+        acc, cm = ctx.mesh_gravity(b, ex, central, 1.0, 0.0, "exact")
+        ref, rcm = orc.vector_field_mesh(b, pairs, ex, central, 1.0, 0.0)
+        assert np.array_equal(bits(acc), bits(ref))
+        if central is not None:
+            assert 0 < np.signbit(ref[:, 2]).sum() < n
+            assert np.array_equal(bits(cm), bits(rcm))
+
+
 @pytest.mark.parametrize("n", [1, 2, 3, 4, 7])
 def test_mesh_gravity_exact_few_bodies(ctx, n):
     b = blob(n, 20 + n, half=0.01)
