@@ -206,7 +206,7 @@ ncg_status ncg_gravity_allpairs_static_dev(ncg_ctx *ctx, const ncg_body *d_bodie
 /* ---------------------------------------------------------------------------
  * Brute-force collision search: replaces brute_force (collision.c:425-456).
  * The GPU tests every pair i<j of existing bodies at the given state with the
- * closest_approach predicate (collision.c:63-172; from 8192 bodies, those pairs
+ * closest_approach predicate (collision.c:63-172; from 12288 bodies, those pairs
  * that the bodies' boxes let meet within the timestep) and hands the candidates to
  * the host, which replays the reference's lexicographic (i, j) order through
  * ops: candidate pairs are confirmed with ops->test and resolved with

@@ -18,7 +18,8 @@
 
 namespace {
 
-// All pairs, upper-triangular tiles of CT bodies, used below NCG_CP_MIN bodies:
+// All pairs, upper-triangular tiles of CT bodies, used below NCG_CP_MIN bodies (by
+// host calls below NCG_CP_HOST_MIN):
 // one workgroup per tile pair, CQ wavefronts that each take CT / CQ of the J
 // tile's bodies against the I tile's (one per lane).  At 2000 bodies it is
 // bound by the length of a wavefront's walk (its tests are few for the chip):
@@ -79,8 +80,6 @@ ncg_status ncg_candidates_launch(ncg_ctx *ctx, const DBody *d_b, int32_t n, cons
                                  double dt, int2 *d_out, unsigned long long cap,
                                  unsigned long long *d_count, hipStream_t st)
 {
-    if (n >= NCG_CP_MIN)
-        return ncg_cp_candidates_launch(ctx, d_b, n, d_ex, dt, d_out, cap, d_count, st);
     const int ntiles = (int)cdiv(n, CT);
     const long nblk = (long)ntiles * (ntiles + 1) / 2;
     if (nblk == 0) return NCG_OK;
@@ -102,7 +101,10 @@ static ncg_status candidates_dev(ncg_ctx *ctx, const DBody *db, int32_t n, const
         unsigned long long *dcnt = dbuf<unsigned long long>(ctx, "cand_cnt", 1);
         if (!dout || !dcnt) return NCG_ERR_NOMEM;
         NCG_HIP(hipMemsetAsync(dcnt, 0, sizeof(unsigned long long), st));
-        const ncg_status r = ncg_candidates_launch(ctx, db, n, dex, dt, dout, cap, dcnt, st);
+        const ncg_status r =
+            n >= NCG_CP_HOST_MIN
+                ? ncg_cp_candidates_launch(ctx, db, n, dex, dt, dout, cap, dcnt, st)
+                : ncg_candidates_launch(ctx, db, n, dex, dt, dout, cap, dcnt, st);
         if (r != NCG_OK) return r;
         unsigned long long cnt = 0;
         NCG_HIP(hipMemcpyAsync(&cnt, dcnt, sizeof cnt, hipMemcpyDeviceToHost, st));

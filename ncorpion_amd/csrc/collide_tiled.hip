@@ -1,5 +1,5 @@
-// Brute-force collision pass over spatial tiles, for one system of CP_MIN
-// bodies and more.
+// Brute-force collision pass over spatial tiles, for one system of NCG_CP_MIN
+// bodies and more (the search alone, for host calls, from NCG_CP_HOST_MIN).
 //
 // The pass has brute_force's results (NcorpiON collision.c:425-456): every
 // pair i < j is a candidate exactly when closest_approach's predicate accepts
@@ -24,6 +24,9 @@
 // changed one and walks the rows between: 13.2 ms for 25 collisions among
 // 65,536 bodies against 0.16 ms here (about 6 us a collision: a chain of dependent
 // loads, the bounce and the two scans).
+//
+// Where every pair is within reach (a timestep in which bodies cross the system)
+// nothing is skipped, and the search takes 1.5 to 1.7 times the tests of all pairs.
 //
 // Nothing here is a library sort or a memset, so the pass can be captured in a
 // graph.

@@ -786,9 +786,11 @@ ncg_status leapfrog_run(ncg_ctx *ctx, ncg_body *d_bodies, int32_t n_in, int32_t 
     // clears it).
     auto collide = [&](double h, bool cleared) -> ncg_status {
         if (!cleared) hipLaunchKernelGGL(k_lf_zero_u64, dim3(1), dim3(1), 0, st, cnt);
-        ncg_status r = ncg_candidates_launch(ctx, b, n, ex, h, cand, cap, cnt, st);
+        const bool tiles = n >= NCG_CP_MIN;
+        ncg_status r = tiles ? ncg_cp_candidates_launch(ctx, b, n, ex, h, cand, cap, cnt, st)
+                             : ncg_candidates_launch(ctx, b, n, ex, h, cand, cap, cnt, st);
         if (r != NCG_OK) return r;
-        if (n >= NCG_CP_MIN)
+        if (tiles)
             return ncg_cp_replay_launch(ctx, b, n, ex, d_did_collide, one_collision_only, cand, cnt,
                                         cap, h, f, stat, st);
         return ncg_bf_replay_launch(ctx, b, ex, d_did_collide, one_collision_only, off, 1, cand,

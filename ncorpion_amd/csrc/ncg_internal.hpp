@@ -180,6 +180,11 @@ ncg_status ncg_candidates_launch(ncg_ctx *ctx, const DBody *d_b, int32_t n, cons
 // 16,384; 192 against 168 at 6000, where the seven launches of the order cost
 // more than they save).
 constexpr int NCG_CP_MIN = 8192;
+// Host calls, whose candidates the host replays, gain only by the search, and wait
+// for its launches: 8192 bodies 122 us a call through the tiles, 97 with all pairs
+// tested; 11,000 150 and 153; 12,288 155 and 174 (clumps 165 and 172); 16,384 180 and
+// 261.
+constexpr int NCG_CP_HOST_MIN = 12288;
 constexpr int NCG_CP_EVENTS = 4096;   // candidates of a pass the tiled replay takes
 constexpr int NCG_CP_CHANGED = 1024;  // bodies changed in a pass it takes (each once)
 constexpr int NCG_CP_FOUND = 2048;    // pairs that the scans of changed bodies may add

@@ -190,6 +190,26 @@ def test_replay_with_removed_and_created_bodies(ctx, seed):
     assert kinds == {0, 1, 2} and ref.largest >= n0  # removals, reuse and appends happened
 
 
+# The search of host calls on both sides of its change from all pairs to tiles: the
+# reference's first hits are among the candidates, and one more absent body, past
+# the change or not, takes only its own pairs away.
+@pytest.mark.parametrize("n", [12287, 12288])
+def test_candidates_on_both_sides_of_the_tiled_search(ctx, n):
+    from ncorpion_amd import ic
+    dt = 0.02
+    b = ic.disk(n, seed=5, mass=1e-8, radius=1e-3)
+    cand = {tuple(p) for p in ctx.collide_candidates(b, None, dt)}
+    _, _, pairs = orc.brute_force(b, dt, 1, 1.5, 0, None)
+    first = {tuple(p) for p in pairs if orc.closest_approach(b, int(p[0]), int(p[1]), dt, None)[0]}
+    assert len(cand) > 20 and first <= cand
+    assert all(orc.closest_approach(b, i, j, dt * (1 + 1e-9), None)[0] for i, j in cand)
+    gone = sorted(cand)[0][0]
+    ex = np.ones(n, np.int32)
+    ex[gone] = 0
+    left = {tuple(p) for p in ctx.collide_candidates(b, ex, dt)}
+    assert left == {p for p in cand if gone not in p}
+
+
 # The limits of the tiled replay: more than 4096 candidates; more than 1024 changed
 # bodies, and just fewer in more than 512 collisions; a clump whose changed bodies
 # have more than 2048 later pairs.  Past a limit the pass is undone and replayed on
