@@ -52,18 +52,19 @@ __device__ inline void exact_term(double X, double Y, double Z, double Rk, doubl
 //
 // What bounds it: from ~5000 bodies the FP64 issue of the terms (44 instructions
 // when the operands are in the window of exact_term.hpp).  Below that neither half
-// alone: of 22 us at 2000 bodies the chain of dependent additions (5.7 clocks each)
+// alone: of 21 us at 2000 bodies the chain of dependent additions (5.7 clocks each)
 // takes 5 and the issue of the terms about 9 (85 instructions a wavefront of them);
 // a wavefront lives 40,000 clocks (counters), 16,000 of them waiting, with two
 // wavefronts a SIMD.  EXP_B = 4 makes the two halves of a chunk about equal (192
 // additions ~1100 clocks, 4 terms ~900).
 // One wavefront per body, its three summing lanes idle during the terms and
 // the other 61 during the sums, took 40 us at 2000 bodies and 2.27 ms at 20,011
-// (and CM_acc 13 and 101 us after it); this form takes 22 us and 1.13 ms with
+// (and CM_acc 13 and 101 us after it); this form takes 21 us and 1.13 ms with
 // CM_acc.  One body per lane, the form above 32,768 bodies before, took 25.7 ms
 // at 65,536 and 212 ms at 262,144, this one 10.9 and 171.  EXP_B = 2 takes 1.66 ms
 // at 20,011 (the summing wavefronts' share), 8 (two workgroups a CU by LDS) 1.17.
 constexpr int EXP_B = 4;
+constexpr int EXP_ACROSS_MAX = 8192; // bodies
 constexpr int EXP_CH = 192;          // bodies j of a chunk
 constexpr int EXP_G = 8;             // pairs of terms the summing lanes read ahead
 constexpr int EXP_RS = EXP_CH + 2;   // row stride: the summing lanes read different banks
@@ -90,34 +91,40 @@ __device__ inline ExpJ exp_load(const DBody *__restrict__ b, int n, const int32_
     return r;
 }
 
-// The window form for EXP_B bodies at once (their chains overlap): for j below
-// (LOWER, negated) or above all of them.  False, with nothing written, when an
-// operand is outside the window.  SOFT false: s is zero; with finite radii the
-// softening is then zero and adds nothing to r2.
-template <bool SOFT, bool LOWER>
+// The window form for EXP_B bodies at once (their chains overlap): for a wavefront
+// of j below all of them (negated), above, or ACROSS, with the bodies themselves
+// among its j.  False, with nothing written, when an operand is outside the window.  SOFT
+// false: s is zero; with finite radii the softening is then zero and adds nothing
+// to r2.
+enum ExpSide { EXP_BELOW, EXP_ABOVE, EXP_ACROSS };
+
+template <bool SOFT, ExpSide SIDE>
 __device__ inline bool exp_window(const ExpJ &q, bool ok, double gm, const double *X,
                                   const double *Y, const double *Z, const double *R, double s,
-                                  double (*row)[EXP_RS], int jl)
+                                  double (*row)[EXP_RS], int jl, int jk /* j - k0 */)
 {
     double t[3][EXP_B], r2[EXP_B];
 #pragma unroll
     for (int u = 0; u < EXP_B; ++u) {
-        t[0][u] = LOWER ? X[u] - q.x : q.x - X[u];
-        t[1][u] = LOWER ? Y[u] - q.y : q.y - Y[u];
-        t[2][u] = LOWER ? Z[u] - q.z : q.z - Z[u];
+        const bool low = SIDE == EXP_BELOW || (SIDE == EXP_ACROSS && jk < u);
+        t[0][u] = low ? X[u] - q.x : q.x - X[u];
+        t[1][u] = low ? Y[u] - q.y : q.y - Y[u];
+        t[2][u] = low ? Z[u] - q.z : q.z - Z[u];
         r2[u] = t[0][u] * t[0][u] + t[1][u] * t[1][u] + t[2][u] * t[2][u];
         if (SOFT) {
             const double soft = s * (R[u] + q.R);
             r2[u] = r2[u] + soft * soft;
         }
-        ok = ok && r2_ok(r2[u]);
+        ok = ok && (r2_ok(r2[u]) || (SIDE == EXP_ACROSS && jk == u));
     }
     if (!__all(ok || q.skip)) return false;
     const bool holes = __any(q.skip);
 #pragma unroll
     for (int u = 0; u < EXP_B; ++u) {
         double v[3] = {gm * t[0][u], gm * t[1][u], gm * t[2][u]};
-        window_quotients<LOWER>(v, r2[u]);
+        window_quotients<SIDE == EXP_BELOW>(v, r2[u]);
+        if (SIDE == EXP_ACROSS)
+            for (int d = 0; d < 3; ++d) v[d] = jk < u ? -v[d] : jk == u ? -0.0 : v[d];
         if (holes && q.skip) v[0] = v[1] = v[2] = -0.0;
 #pragma unroll
         for (int d = 0; d < 3; ++d) row[3 * u + d][jl] = v[d];
@@ -125,7 +132,11 @@ __device__ inline bool exp_window(const ExpJ &q, bool ok, double gm, const doubl
     return true;
 }
 
-template <bool SOFT>
+// ACROSS: the one wavefront of terms with the bodies themselves among its j takes the
+// window form too (64 bodies: 4.7 us a call, 5.6 with the form with branches; 2000: a
+// resident step 2 % less).  With many other wavefronts it gains nothing, and the
+// larger loop costs (32,000 bodies: 2.97 ms against 2.94).
+template <bool SOFT, bool ACROSS>
 __global__ __launch_bounds__(256) void k_grav_exact_p(const DBody *__restrict__ b, int n,
                                                       const int32_t *__restrict__ ex, int cp,
                                                       double cx, double cy, double cz, double mu,
@@ -194,12 +205,20 @@ __global__ __launch_bounds__(256) void k_grav_exact_p(const DBody *__restrict__ 
                 for (int d = 0; d < 3; ++d) row[d][jl] = t[d];
             } else {
                 const int j0 = c * EXP_CH + (w - 1) * 64;
-                const bool ok = kok && coord_ok(now.x) && coord_ok(now.y) && coord_ok(now.z) &&
-                                gm_ok(gm) && (SOFT || fabs(now.R) < 1e100);
+                // Zeros are looked for only where there is something else (1 % of the
+                // kernel at 20,011 bodies).
+                bool ok = kok && coord_big(now.x) && coord_big(now.y) && coord_big(now.z) &&
+                          gm_big(gm) && (SOFT || fabs(now.R) < 1e100);
+                if (!__all(ok || now.skip))
+                    ok = kok && coord_ok(now.x) && coord_ok(now.y) && coord_ok(now.z) && gm_ok(gm) &&
+                         (SOFT || fabs(now.R) < 1e100);
                 bool done = false;
-                if (j0 + 63 < k0) done = exp_window<SOFT, true>(now, ok, gm, X, Y, Z, R, s, row, jl);
+                if (j0 + 63 < k0)
+                    done = exp_window<SOFT, EXP_BELOW>(now, ok, gm, X, Y, Z, R, s, row, jl, j - k0);
                 else if (j0 >= k0 + EXP_B)
-                    done = exp_window<SOFT, false>(now, ok, gm, X, Y, Z, R, s, row, jl);
+                    done = exp_window<SOFT, EXP_ABOVE>(now, ok, gm, X, Y, Z, R, s, row, jl, j - k0);
+                else if (ACROSS)
+                    done = exp_window<SOFT, EXP_ACROSS>(now, ok, gm, X, Y, Z, R, s, row, jl, j - k0);
                 if (!done) {
 #pragma nounroll
                     for (int u = 0; u < EXP_B; ++u) {
@@ -296,12 +315,13 @@ static ncg_status exact_launch(ncg_ctx *ctx, const DBody *d_b, int32_t n, const 
     const double mu = cp ? G * c->mass : 0.0;  // physics.c:131
     const int cmblk = d_cm_acc ? 1 : 0;
     const dim3 grid(cmblk + cdiv(n, EXP_B));
-    if (soft != 0.0)
-        hipLaunchKernelGGL(k_grav_exact_p<true>, grid, dim3(256), 0, st, d_b, (int)n, d_ex, cp, cx,
-                           cy, cz, mu, d_cen, G, soft, d_init, d_acc, cmblk, d_cm_acc, tail);
-    else
-        hipLaunchKernelGGL(k_grav_exact_p<false>, grid, dim3(256), 0, st, d_b, (int)n, d_ex, cp, cx,
-                           cy, cz, mu, d_cen, G, soft, d_init, d_acc, cmblk, d_cm_acc, tail);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, d_b, (int)n, d_ex, cp, cx, cy, cz, mu,
+                           d_cen, G, soft, d_init, d_acc, cmblk, d_cm_acc, tail);
+    };
+    if (n <= EXP_ACROSS_MAX) soft != 0.0 ? launch(k_grav_exact_p<true, true>)
+                                         : launch(k_grav_exact_p<false, true>);
+    else soft != 0.0 ? launch(k_grav_exact_p<true, false>) : launch(k_grav_exact_p<false, false>);
     NCG_CHECK_LAUNCH();
     return NCG_OK;
 }

@@ -252,6 +252,19 @@ def test_exact_bitwise_edges(ctx, n, kind, soft):
         assert np.array_equal(bits(cm), bits(rcm))
 
 
+# Both sides of the change between the two instances of the exact kernel (8192 bodies):
+# rows at the edges of chunks and workgroups, bit for bit.
+@pytest.mark.parametrize("n", [8192, 8193])
+def test_exact_rows_on_both_sides_of_8192(ctx, n):
+    m, R = ic.disk_c3_masses(n, n)
+    b = ic.disk(n, seed=n, masses=m, radii=R)
+    rows = np.array([0, 3, 4, 63, 64, 191, 192, 4095, 8127, 8128, n - 2, n - 1])
+    for soft in (0.0, 1e-3):
+        ref = orc.vector_field_rows(b, rows, None, (1e-3, 0.0, 0.0, 1.0), 1.0, soft)
+        acc, _ = ctx.gravity_allpairs(b, None, (1e-3, 0.0, 0.0, 1.0), 1.0, soft, "exact")
+        assert np.array_equal(bits(acc[rows]), bits(ref))
+
+
 # Massless and negative bodies are in the window: their terms' zeros and signs.
 @pytest.mark.parametrize("n", [65, 193, 577])
 def test_exact_massless_and_negative_bodies(ctx, n):
